@@ -56,6 +56,20 @@ constexpr int kTablePadRows = 7;
 // inside the buffer.
 constexpr int kTableGuardRows = 16;
 
+// Layouts of the expanded tables: `lane_cells` 0, rows of W taps with the pad
+// rows above and below (the kernels that read whole chunks of grid rows); 1
+// or 2, no pad rows, each row filled up with zeros to whole units of 8 or 16
+// taps (at least one zero in the latter), for the band kernel, whose lanes
+// take that many adjacent taps.
+__host__ __device__ __forceinline__ int table_stride(int W, int lane_cells)
+{
+    return lane_cells == 2 ? (W + 16) / 16 * 16 : lane_cells == 1 ? (W + 7) / 8 * 8 : W;
+}
+__host__ __device__ __forceinline__ int table_pad_rows(int lane_cells)
+{
+    return lane_cells ? 0 : kTablePadRows;
+}
+
 __device__ __forceinline__ int meta_support(int packed) { return (packed >> kSupportShift) & 0xFFF; }
 __device__ __forceinline__ unsigned meta_table_id(int packed) { return (unsigned)packed >> kTableIdShift; }
 
@@ -84,6 +98,7 @@ struct JobDev
     unsigned tile_base;        // first global tile id of this job
     unsigned long long vis_begin, vis_end;
     unsigned chunk_base;       // first selection chunk of this job
+    unsigned visits_per_item;  // tile visits per work item
 };
 
 // Selection constants of a job in the selection precision.

@@ -10,7 +10,8 @@
 //   radix sort       stable LSD sort of the pairs by key
 //   k_tile_bounds    first/last visit of each tile in sorted order
 //   k_items / scan / k_item_map   split tiles into work items
-//   k_grid_tiles     one workgroup per work item, tile in registers (or LDS)
+//   k_grid_tiles     one workgroup per work item, tile in registers (or LDS);
+//                    k_grid_strips, k_grid_staged, k_grid_bands: own headers
 //   k_merge          ordered FP64 sum of partial tiles into the grid
 //   k_degrid         adjoint: one wave per visibility, taps dealt to all lanes
 #pragma once
@@ -29,8 +30,8 @@ namespace gg {
 // stores that tap at row j + s, column k + s, a dense (2s+1)^2 complex
 // array: a wave reads one contiguous 512-byte row segment.  Negative offsets
 // use the same table mirrored (|-a + ov*k| = |a + ov*(-k)|).  Each table
-// occupies (W + 2*kTablePadRows) rows of W taps, the pad rows zero; the
-// table's row 0 sits kTablePadRows rows into its block.
+// occupies (W + 2*table_pad_rows) rows of table_stride taps, the padding
+// zero; the table's row 0 sits table_pad_rows rows into its block.
 // TI: precision of the caller's kernel stack; TA: precision the gridder
 // accumulates in (the tables are stored in TA; float -> double is exact).
 // One wave per table row (pad rows included): the row's table and row index
@@ -42,35 +43,37 @@ __global__ __launch_bounds__(256)
 void k_expand_tables(const typename V2<TI>::t* __restrict__ conv,
         int num_planes, int conv_size_half, int oversample, int half_ov,
         const int* __restrict__ support, const unsigned* __restrict__ plane_off,
-        typename V2<TA>::t* __restrict__ tables)
+        int lane_cells, typename V2<TA>::t* __restrict__ tables)
 {
     const size_t plane_len = (size_t)conv_size_half * conv_size_half;
     const int noff = half_ov + 1;
+    const int pad = table_pad_rows(lane_cells);
     const int lane = lane_id();
     const int wave = (int)(threadIdx.x >> 6), waves = (int)(blockDim.x >> 6);
     for (int p = blockIdx.y; p < num_planes; p += gridDim.y)
     {
         const int s = support[p];
         const int W = 2 * s + 1;
-        const int rows = W + 2 * kTablePadRows;          // rows of one padded table
+        const int stride = table_stride(W, lane_cells);
+        const int rows = W + 2 * pad;                    // rows of one padded table
         const int total_rows = rows * noff * noff;
         const typename V2<TI>::t* src = conv + plane_len * p;
         typename V2<TA>::t* dst = tables + plane_off[p];
         for (int rr = blockIdx.x * waves + wave; rr < total_rows; rr += gridDim.x * waves)
         {
             const int tab = rr / rows;
-            const int jj = rr - tab * rows - kTablePadRows;
+            const int jj = rr - tab * rows - pad;
             const int a = tab / noff, b = tab - a * noff;
-            typename V2<TA>::t* out = dst + (size_t)rr * W;
+            typename V2<TA>::t* out = dst + (size_t)rr * stride;
             const bool in = jj >= 0 && jj < W;
             const typename V2<TI>::t* srow =
                     src + (in ? (size_t)abs(b + oversample * (jj - s)) * conv_size_half : 0);
-            for (int kk = lane; kk < W; kk += 64)
+            for (int kk = lane; kk < stride; kk += 64)
             {
                 typename V2<TA>::t o;
                 o.x = (TA)0;
                 o.y = (TA)0;
-                if (in)
+                if (in && kk < W)
                 {
                     const typename V2<TI>::t v = srow[abs(a + oversample * (kk - s))];
                     o.x = (TA)v.x;
@@ -131,13 +134,13 @@ constexpr int kSelPerThread = 4;
 constexpr int kSelChunk = kSelThreads * kSelPerThread;   // visibilities per chunk
 
 // A visibility's record and weighted amplitude side by side (32 bytes), for
-// the strip kernel's gather, which reads them in sorted-visit order, that is
-// at random: one 32-byte read instead of two 16-byte ones.
+// the strip and band kernels' gathers, which read them in sorted-visit order,
+// that is at random: one 32-byte read instead of two.
+template <typename T>
 struct __align__(32) VisRec
 {
     int4 meta;
-    float2 amp;                      // weight * vis (re, im)
-    float2 pad;
+    typename V2<T>::t amp;           // weight * vis (re, im)
 };
 
 template <typename TI, typename TA>
@@ -150,9 +153,10 @@ struct SelectArgs
     const double* norm_table; const unsigned* plane_off;
     int table_id_shift;              // table id >> shift fits kTableIdBits
     int tw, th;                      // bucketing tile width / height (cells)
+    int lane_cells;                  // layout of the expanded tables
     // outputs
     int4* meta; typename V4<TA>::t* amp; unsigned* num_visits;
-    VisRec* vrec;                    // FP32 strip path: meta and (re, im) in one record, or null
+    VisRec<TA>* vrec;                // strip and band paths: meta and (re, im) in one record, or null
     double* part_norm; unsigned long long* part_skipped;
     unsigned long long* part_taps; unsigned long long* part_nonfinite; int4* part_bbox;
 };
@@ -263,8 +267,8 @@ void k_select(const SelectArgs<TI, TA> A, unsigned num_chunks)
                 amp_re = v_re;
                 amp_im = v_im;
                 const bool nonfinite = !isfinite(v_re) || !isfinite(v_im);
-                // (the strip path reads amplitudes from vrec; only the
-                // non-finite pass reads amp there)
+                // (the strip and band paths read amplitudes from vrec; only
+                // the non-finite pass reads amp there)
                 if (!A.vrec || nonfinite) A.amp[i] = am;
                 if (nonfinite)
                 {
@@ -274,19 +278,16 @@ void k_select(const SelectArgs<TI, TA> A, unsigned num_chunks)
             }
             m.z = (int)(((table_id >> A.table_id_shift) << kTableIdShift) |
                     ((unsigned)s.support << kSupportShift) | (unsigned)flags);
-            m.w = (int)(A.plane_off[s.plane] + tab * (unsigned)(W + 2 * kTablePadRows) * (unsigned)W +
-                    (unsigned)(kTablePadRows * W));
+            const unsigned pad = (unsigned)table_pad_rows(A.lane_cells);
+            const unsigned stride = (unsigned)table_stride(W, A.lane_cells);
+            m.w = (int)(A.plane_off[s.plane] + tab * ((unsigned)W + 2 * pad) * stride + pad * stride);
             A.meta[i] = m;
-            if constexpr (std::is_same<TA, float>::value)
+            if (A.vrec)
             {
-                if (A.vrec)
-                {
-                    VisRec rr;
-                    rr.meta = m;
-                    rr.amp = make_float2(amp_re, amp_im);
-                    rr.pad = make_float2(0.f, 0.f);
-                    A.vrec[i] = rr;
-                }
+                VisRec<TA> rr;
+                rr.meta = m;
+                rr.amp = {amp_re, amp_im};
+                A.vrec[i] = rr;
             }
             // Tile visits (none for non-finite amplitudes: k_grid_nonfinite
             // grids those after the tiles are done).
@@ -811,7 +812,7 @@ __global__ void k_run_starts(const unsigned* __restrict__ flag,
 // vlds the visit's part of its staged LDS offsets.
 template <typename T>
 __global__ void k_gather_visits(const unsigned* __restrict__ vals,
-        const VisRec* __restrict__ vrec,
+        const VisRec<T>* __restrict__ vrec,
         const unsigned* __restrict__ run_flag, const unsigned* __restrict__ run_excl,
         const unsigned* __restrict__ run_start, uint4 min_run, int max_w, int lds_stride,
         const unsigned* __restrict__ keys, int key_table_bits,
@@ -826,7 +827,7 @@ __global__ void k_gather_visits(const unsigned* __restrict__ vals,
             p < n; p += (unsigned long long)gridDim.x * blockDim.x)
     {
         const unsigned i = vals[p];
-        const VisRec rec = vrec[i];
+        const VisRec<T> rec = vrec[i];
         int4 m = rec.meta;
         const unsigned r = run_excl[p] + run_flag[p] - 1u;
         const int W = 2 * meta_support(m.z) + 1;
@@ -871,18 +872,23 @@ __global__ void k_gather_visits(const unsigned* __restrict__ vals,
     }
 }
 
-// Work items per tile: ceil(visits / visits_per_item); tiles with two or more
-// items also take that many partial-tile slots.
+// Work items per tile: ceil(visits / visits_per_item) with the job's item size
+// (or `override` where that is not 0); tiles with two or more items also take
+// that many partial-tile slots.
+template <typename T>
 __global__ void k_items(const unsigned* __restrict__ tile_start,
         const unsigned* __restrict__ tile_end, unsigned num_tiles,
-        unsigned visits_per_item, unsigned* __restrict__ n_items,
+        const JobDev<T>* __restrict__ jobs, const unsigned* __restrict__ job_tile_base,
+        int num_jobs, unsigned override, unsigned* __restrict__ n_items,
         unsigned* __restrict__ n_slots)
 {
     for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < num_tiles;
             t += gridDim.x * blockDim.x)
     {
         const unsigned cnt = tile_end[t] - tile_start[t];
-        const unsigned ni = (cnt + visits_per_item - 1) / visits_per_item;
+        const unsigned vpi = override ? override
+                                      : jobs[find_job(job_tile_base, num_jobs, t)].visits_per_item;
+        const unsigned ni = (cnt + vpi - 1) / vpi;
         n_items[t] = ni;
         n_slots[t] = ni >= 2 ? ni : 0u;
     }
@@ -899,6 +905,8 @@ __global__ void k_item_map(const unsigned* __restrict__ item_off, unsigned num_t
 // ===========================================================================
 // Gridding
 // ===========================================================================
+template <typename T> struct BandItem;
+
 template <typename T>
 struct GridArgs
 {
@@ -921,10 +929,11 @@ struct GridArgs
     const unsigned* run_start; const int* run_z; const int* run_tb;
     const unsigned long long* d_num_runs;
     unsigned min_stage_run;        // shortest run staged through LDS
-    const int4* vmeta;             // meta / amp of each sorted visit (strip kernel)
+    const int4* vmeta;             // records of each sorted visit (strip and band kernels)
     const typename V2<T>::t* vamp;        // weighted amplitude per sorted visit
     const int* vlds;               // per sorted visit: its part of the staged LDS offsets
-    unsigned item_group;           // strip kernel: consecutive items per XCD (>= 1)
+    unsigned item_group;           // strip and band kernels: consecutive items per XCD (>= 1)
+    const struct BandItem<T>* band_items;   // band kernel: its items, in the order they are taken
     unsigned* item_ctr;            // strip kernel: 8 zeroed counters (positions
                                    // taken per XCD)
 };
@@ -1237,7 +1246,8 @@ __global__ __launch_bounds__(256)
 void k_grid_nonfinite(const typename V2<T>::t* __restrict__ tables,
         const int4* __restrict__ meta, const typename V4<T>::t* __restrict__ amp,
         const JobDev<T>* __restrict__ jobs, const unsigned long long* __restrict__ job_vis_off,
-        int num_jobs, unsigned long long n, const unsigned long long* __restrict__ job_out)
+        int num_jobs, unsigned long long n, const unsigned long long* __restrict__ job_out,
+        int lane_cells)
 {
     typedef typename V2<T>::t T2;
     const int lane = lane_id();
@@ -1262,11 +1272,11 @@ void k_grid_nonfinite(const typename V2<T>::t* __restrict__ tables,
         const JobDev<T> J = ld_const(jobs, lo);
         const typename V4<T>::t a = ld_const(amp, i);
         const int s = meta_support(mt.z);
-        const int W = 2 * s + 1;
+        const int stride = table_stride(2 * s + 1, lane_cells);
         const bool neg_u = mt.z & kFlagNegU, neg_v = mt.z & kFlagNegV;
         for (int jr = -s; jr <= s; ++jr)
         {
-            const T2* krow = tables + (unsigned)mt.w + (neg_v ? s - jr : s + jr) * W;
+            const T2* krow = tables + (unsigned)mt.w + (neg_v ? s - jr : s + jr) * stride;
             T* grow = reinterpret_cast<T*>(J.grid + (size_t)(mt.y + jr) * J.grid_size + mt.x);
             for (int k = -s + lane; k <= s; k += 64)
             {

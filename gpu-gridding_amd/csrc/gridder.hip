@@ -7,6 +7,7 @@
 #include "gg_kernels.hpp"
 #include "gg_grid_staged.hpp"
 #include "gg_grid_strips.hpp"
+#include "gg_grid_bands.hpp"
 #include "gg_weights.hpp"
 #include "gg_image.hpp"
 #include "gg_status.hpp"
@@ -215,16 +216,17 @@ struct mi355_ctx
     // stats_in_noalloc is set.
     mi355_ctx* noalloc_ctx = nullptr;
     bool stats_in_noalloc = false;
-    // the last strip-kernel pass's sorted tile lists (mi355_ctx_get_buckets)
-    bool bk_valid = false;
+    // the last strip- or band-kernel FP32 pass's sorted tile lists (mi355_ctx_get_buckets)
+    bool bk_valid = false, bk_bands = false, bk_exact = false;
     int bk_cur = 0, bk_key_table_bits = 0;
+    unsigned long long bk_points = 0;
     unsigned long long bk_count = 0;
     unsigned char* arena = nullptr;
     size_t arena_cap = 0, arena_used = 0;
 
     // prepared kernel tables
     const void* cache_conv = nullptr;
-    int cache_prec = 0, cache_ov = 0, cache_csh = 0;
+    int cache_prec = 0, cache_ov = 0, cache_csh = 0, cache_lane_cells = 0;
     std::vector<int> cache_support;
     bool tables_valid = false;
     std::vector<unsigned> plane_off;
@@ -239,8 +241,9 @@ struct mi355_ctx
     DevBuf keys[2], vals[2], hist, hist_off;
     DevBuf tile_start, tile_end, n_items, n_slots, item_off, slot_off, item_tile;
     DevBuf run_start, run_z, run_tb;
-    DevBuf vmeta, vamp, vlds;       // sorted visit records (strip kernel)
-    DevBuf vrec;                    // per-visibility record + amplitude (strip kernel's gather)
+    DevBuf vmeta, vamp, vlds;       // sorted visit records (strip and band kernels)
+    DevBuf vrec;                    // per-visibility record + amplitude (their gathers)
+    DevBuf band_items, order_count; // band kernel: its items, and their counts by first table
     DevBuf scratch;
     DevBuf jobs_d, job_chunk_off_d, job_vis_off_d, job_tile_base_d, job_out_d, job_bbox_d, job_norm_d;
     // drop-in staging
@@ -305,6 +308,80 @@ unsigned auto_visits_per_item(unsigned long long num_points, int num_cu)
 // table pays only over longer runs (support-72 shape: 255.4 ms at 3, 241.8
 // ms at 8; 2.15M-visibility shape 17.0 -> 15.3 ms).
 unsigned stage_run_default(bool fp64_tiles) { return fp64_tiles ? 8u : 3u; }
+
+// Band kernel: visits per work item.  An item is worked on by 32 waves, one
+// per band of 8 rows and column block, so a small call needs small items to
+// fill the chip (kernel and merge, 2,003 visibilities: 157 us with items of
+// 1024 visits, 38 us with 64; 200,000: 269 us with 1024, 221 us with 512),
+// a large one fewer partial regions to merge (13.2M in 24 grids: 23.7 ms with
+// 512, 23.0 ms with 1024, 23.9 ms with 2048).  Up to 65,536 visibilities the
+// size keeps the partial regions below about 200 (50 MiB).
+unsigned band_visits_per_item(unsigned long long num_points)
+{
+    if (num_points > 65536)
+        return num_points < 524288 ? 512u : num_points < (16ull << 20) ? 1024u : 4096u;
+    unsigned v = 64;
+    while (v * 128ull < num_points) v <<= 1;
+    return v;
+}
+// Visibilities from which the band kernel's items go in table order.
+constexpr unsigned long long kBandOrderMin = 524288;
+
+// Elements of the expanded tables of all planes, guards not counted.
+unsigned long long table_elements(size_t P, const int* support, int ov, int lane_cells)
+{
+    const unsigned long long noff = (ov + 1) / 2 + 1, pad = 2ull * table_pad_rows(lane_cells);
+    unsigned long long n = 0;
+    for (size_t p = 0; p < P; ++p)
+    {
+        const int W = 2 * support[p] + 1;
+        n += ((unsigned long long)W + pad) * (unsigned long long)table_stride(W, lane_cells) * noff * noff;
+    }
+    return n;
+}
+
+// Whether the band kernel takes a pass (tiles: regions of 256 x 128 cells in
+// all its grids).  Not where another kernel or a staging threshold is asked
+// for.  FP64: always (1.13 to 3.3 times the 64x64 staged kernel's speed at
+// supports 16 to 72, 0.2M to 12M visibilities, 32 and 300 planes, 2048^2 and
+// 8192^2 grids).  FP32: where tables serve few visits or are small; the strip
+// kernel, which stages a table once for many visits, stays ahead with wide
+// tables on large grids (support 72: 0.86 to 0.96 of its time at 1M to 8M
+// visibilities and 16384^2, but 1.02 to 1.57 times its speed at 2048^2; support
+// 48 and below: 1.0 to 2.3 times) and where a table serves tens of thousands
+// (support 48, 12M visibilities, 32 planes, 8192^2: 0.88).  Compensated FP32
+// has FP64 cells here and so half the cells a lane: ahead up to the visits
+// per table below (1M visibilities, 128 planes, support 32: 1.58 + 0.16 ms
+// before, 1.36 + 0.08 ms).
+template <typename T>
+bool use_bands(const mi355_ctx* C, size_t P, const int* support, int ov, unsigned long long points,
+        unsigned long long tiles)
+{
+    constexpr bool f32 = std::is_same<T, float>::value;
+    if (C->grid_kernel != 0 || C->min_stage_run || C->msr_class[0] || C->msr_class[1] ||
+            C->msr_class[2] || C->msr_class[3])
+        return false;
+    const bool comp = f32 && C->compensated;
+    // Under a workspace cap or in the static scratch a call must not need
+    // more than it did: FP64 keeps its kernel there, FP32 (whose items fall
+    // back to the strip kernel's size) unless the tables grow.  Nor do tables
+    // near the 2 GiB limit.
+    const int lane_cells = f32 && !comp ? 2 : 1;
+    const unsigned long long now = table_elements(P, support, ov, lane_cells);
+    const unsigned long long other = table_elements(P, support, ov, 0);
+    if ((C->max_workspace || C->arena) && (!f32 || comp || now > other)) return false;
+    if (now > other && now * 2 * sizeof(T) > 0x7F000000ull) return false;
+    if (!f32) return true;
+    int smax = 0;
+    for (size_t p = 0; p < P; ++p) smax = std::max(smax, support[p]);
+    const unsigned long long noff = (ov + 1) / 2 + 1;
+    const unsigned long long per_table = points / ((unsigned long long)P * noff * noff);
+    if (comp)
+        return per_table < (smax <= 16 ? 16384u : smax <= 36 ? 2048u : smax <= 48 ? 512u
+                            : smax <= 72 ? 128u : 0u);
+    if (tiles < 1024) return true;
+    return !(smax > 48 && points >= 1000000) && !(smax > 16 && per_table > 20000);
+}
 
 // The strip kernel's thresholds per support class (tables at most 33, 65,
 // 97, 111 wide): the class option, else the option for all classes, else
@@ -389,6 +466,15 @@ int ensure(mi355_ctx* C, DevBuf& b, size_t bytes)
     return MI355_OK;
 }
 
+// Whether buffer b could hold `bytes` within the static scratch or the
+// workspace cap (a context without either: always).
+bool fits(const mi355_ctx* C, const DevBuf& b, size_t bytes)
+{
+    if (bytes <= b.cap) return true;
+    if (C->arena) return C->arena_used + 256 + bytes <= C->arena_cap;
+    return !C->max_workspace || C->ws_bytes - b.cap + bytes <= C->max_workspace;
+}
+
 void release(mi355_ctx* C, DevBuf& b)
 {
     if (C->arena)        // (a view into the static scratch: nothing to free)
@@ -458,7 +544,8 @@ std::vector<DevBuf*> device_buffers(mi355_ctx* C)
         &C->jobs_d, &C->job_chunk_off_d, &C->job_vis_off_d, &C->job_tile_base_d,
         &C->job_out_d, &C->job_bbox_d, &C->job_norm_d, &C->in_conv, &C->in_uu, &C->in_vv, &C->in_ww,
         &C->in_vis, &C->in_weight, &C->in_grid, &C->in_norm, &C->in_skipped, &C->in_weight_out,
-        &C->fft_work, &C->in_image, &C->vmeta, &C->vamp, &C->vlds, &C->vrec};
+        &C->fft_work, &C->in_image, &C->vmeta, &C->vamp, &C->vlds, &C->vrec,
+        &C->band_items, &C->order_count};
 }
 
 int get_default_ctx(mi355_ctx** out)
@@ -520,11 +607,12 @@ int check_grid_args(int grid_size)
 // ---------------------------------------------------------------------------
 template <typename TI, typename TA>
 int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
-        const typename V2<TI>::t* conv_dev)
+        const typename V2<TI>::t* conv_dev, int lane_cells)
 {
     const int prec = (int)(16 * sizeof(TI) + sizeof(TA));
     if (!C->sync_free && C->cache_kernels && C->tables_valid && C->cache_conv == conv_dev &&
             C->cache_prec == prec && C->cache_ov == ov && C->cache_csh == csh &&
+            C->cache_lane_cells == lane_cells &&
             C->cache_support.size() == P &&
             std::equal(support, support + P, C->cache_support.begin()))
         return MI355_OK;
@@ -543,8 +631,7 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     for (size_t p = 0; p < P; ++p)
     {
         C->plane_off[p] = (unsigned)off;
-        const unsigned long long W = 2ull * support[p] + 1;
-        off += (W + 2 * kTablePadRows) * W * noff * noff;
+        off += table_elements(1, support + p, ov, lane_cells);
         if (off > 0x7FFFFFFFull)
             return fail(MI355_ERR_TOO_LARGE, "expanded kernel tables exceed 2^31 elements");
     }
@@ -578,11 +665,11 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     }
     {
         // four rows (waves) per workgroup, at most 16 workgroups per plane
-        const unsigned rows_max = (unsigned)((Wmax + 2 * kTablePadRows) * noff * noff);
+        const unsigned rows_max = (unsigned)((Wmax + 2 * table_pad_rows(lane_cells)) * noff * noff);
         dim3 g(grid_blocks(rows_max, 4, 16), (unsigned)std::min<size_t>(P, 65535));
         hipLaunchKernelGGL((k_expand_tables<TI, TA>), g, dim3(256), 0, C->stream,
                 conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-                C->plane_off_d.as<unsigned>(), C->tables.as<T2>());
+                C->plane_off_d.as<unsigned>(), lane_cells, C->tables.as<T2>());
         HIP_TRY(hipGetLastError());
         const unsigned entries = (unsigned)(P * noff * noff);   // (|off_u|, |off_v|) per plane
         hipLaunchKernelGGL(k_norm_table<TI>, dim3(grid_blocks(entries, 4, 65535)), dim3(256), 0,
@@ -594,6 +681,7 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     C->cache_prec = prec;
     C->cache_ov = ov;
     C->cache_csh = csh;
+    C->cache_lane_cells = lane_cells;
     C->tables_valid = true;
     return MI355_OK;
 }
@@ -687,7 +775,7 @@ struct JobHost
 // gridded after the tiled path on the same stream.
 template <typename T>
 int grid_nonfinite(mi355_ctx* C, unsigned long long count, int num_jobs,
-        unsigned long long n_total)
+        unsigned long long n_total, int lane_cells)
 {
     if (!count) return MI355_OK;
     typedef typename V2<T>::t T2;
@@ -695,7 +783,7 @@ int grid_nonfinite(mi355_ctx* C, unsigned long long count, int num_jobs,
     hipLaunchKernelGGL(k_grid_nonfinite<T>, dim3(grid_blocks(n_total, 4, 65535)), dim3(256), 0,
             C->stream, C->tables.as<T2>(), C->meta.as<int4>(), C->amp.as<T4>(),
             C->jobs_d.as<JobDev<T>>(), C->job_vis_off_d.as<unsigned long long>(), num_jobs,
-            n_total, C->job_out_d.as<unsigned long long>());
+            n_total, C->job_out_d.as<unsigned long long>(), lane_cells);
     HIP_TRY(hipGetLastError());
     return MI355_OK;
 }
@@ -720,6 +808,22 @@ struct BeforeGrid
     virtual ~BeforeGrid() {}
 };
 
+// use_bands for a job table: by the largest job, so that a batched pass grids
+// a job as a call of its own would.
+template <typename TI, typename TA>
+bool auto_kernel_is_bands(const mi355_ctx* C, size_t P, const int* support, int ov, int num_jobs,
+        const JobHost<TI, TA>* jobs)
+{
+    unsigned long long points = 0, regions = 0;
+    for (int j = 0; j < num_jobs; ++j)
+    {
+        const unsigned long long G = (unsigned long long)std::max(jobs[j].grid_size, 0);
+        points = std::max(points, jobs[j].num_points);
+        regions = std::max(regions, ((G + 255) / 256) * ((G + 127) / 128));
+    }
+    return use_bands<TA>(C, P, support, ov, points, regions);
+}
+
 template <typename TI, typename TA>
 int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         const typename V2<TI>::t* conv, int num_jobs, const JobHost<TI, TA>* jobs,
@@ -734,19 +838,27 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     C->stats_in_noalloc = false;
     C->bk_valid = false;
     record(C, EV_START);
-    TRY((prepare_tables<TI, TA>(C, P, support, ov, csh, conv)));
-    record(C, EV_PREP);
     const int half = (ov + 1) / 2, noff = half + 1;
-    // Gridding kernel and bucketing geometry: FP32 uses the strip kernel on
-    // 256 x 128 regions (compensated: 192 x 64) unless another kernel is
-    // asked for; the 64 x 64 kernels take every other case.
+    // Gridding kernel and bucketing geometry, unless a kernel is asked for:
+    // the band kernel where use_bands says so; for FP32 otherwise the strip
+    // kernel on 256 x 128 regions (compensated: 192 x 64); the 64 x 64
+    // kernels take every other case.
+    constexpr bool f32 = std::is_same<T, float>::value;
     const bool comp = C->compensated;
-    const bool strips = std::is_same<T, float>::value && C->grid_kernel == 0;
+    const bool bands = auto_kernel_is_bands(C, P, support, ov, num_jobs, jobs);
+    const bool strips = f32 && C->grid_kernel == 0 && !bands;
+    // (compensated FP32: the band kernel's cells are FP64)
+    using BandPlain = BandCfg<T, T>;
+    using BandComp = BandCfg<T, double>;
+    const bool wide = comp && f32;
+    const int lane_cells = !bands ? 0 : wide ? BandComp::kLaneCells : BandPlain::kLaneCells;
+    TRY((prepare_tables<TI, TA>(C, P, support, ov, csh, conv, lane_cells)));
+    record(C, EV_PREP);
     // (the direct 64 x 64 kernel launches one workgroup per item: not in the
     // host-sync-free mode, which takes the staged one instead)
     const bool direct64 = !strips && C->grid_kernel == 1 && !C->sync_free;
-    const int tw = strips ? (comp ? StripComp::kRegionW : StripPlain::kRegionW) : kTileW;
-    const int th = strips ? (comp ? StripComp::kRegionH : StripPlain::kRegionH) : kTileH;
+    const int tw = bands ? (wide ? BandComp::kRegionW : BandPlain::kRegionW) : strips ? (comp ? StripComp::kRegionW : StripPlain::kRegionW) : kTileW;
+    const int th = bands ? BandPlain::kRegionH : strips ? (comp ? StripComp::kRegionH : StripPlain::kRegionH) : kTileH;
 
     // Jobs.
     C->h_jobs.resize(sizeof(JobDev<T>) * num_jobs);
@@ -779,6 +891,9 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         d.vis_begin = n_total;
         d.vis_end = n_total + J.num_points;
         d.chunk_base = (unsigned)chunks;
+        // (the band kernel's own size; the others' is known once the visit
+        // count is, and overrides it)
+        d.visits_per_item = band_visits_per_item(J.num_points);
         hj[j] = d;
         C->h_job_chunk_off[j] = (unsigned)chunks;
         C->h_job_tile_base[j] = (unsigned)tiles;
@@ -801,9 +916,9 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // Sort key: tile, then the table id as the visit records hold it, then
     // (64x64 staged kernels, which stage a table already mirrored) the two
     // orientation bits; the strip kernel mirrors when reading LDS, so its
-    // runs span orientations.  Low bits are dropped if the key exceeds 32
-    // bits.
-    const int orient_bits = strips ? 0 : 2;
+    // runs span orientations (and the band kernel has none).  Low bits are
+    // dropped if the key exceeds 32 bits.
+    const int orient_bits = strips || bands ? 0 : 2;
     const int table_bits_full = bits_for(num_tables);
     const int table_id_shift = std::max(0, table_bits_full - kTableIdBits);
     const int kappa_bits = table_bits_full - table_id_shift + orient_bits;
@@ -828,7 +943,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // Selection.
     TRY(ensure(C, C->meta, n_total * sizeof(int4)));
     TRY(ensure(C, C->amp, n_total * sizeof(T4)));
-    if (strips) TRY(ensure(C, C->vrec, n_total * sizeof(VisRec)));
+    if (strips || bands) TRY(ensure(C, C->vrec, n_total * sizeof(VisRec<T>)));
     TRY(ensure(C, C->num_visits, n_total * sizeof(unsigned)));
     TRY(ensure(C, C->visit_off, (n_total + 1) * sizeof(unsigned)));
     TRY(ensure(C, C->part_norm, chunks * sizeof(double)));
@@ -851,8 +966,9 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     sa.plane_off = C->plane_off_d.as<unsigned>();
     sa.table_id_shift = table_id_shift;
     sa.tw = tw; sa.th = th;
+    sa.lane_cells = lane_cells;
     sa.meta = C->meta.as<int4>(); sa.amp = C->amp.as<T4>();
-    sa.vrec = strips ? C->vrec.as<VisRec>() : nullptr;
+    sa.vrec = strips || bands ? C->vrec.as<VisRec<T>>() : nullptr;
     sa.num_visits = C->num_visits.as<unsigned>();
     sa.part_norm = C->part_norm.as<double>();
     sa.part_skipped = C->part_skipped.as<unsigned long long>();
@@ -886,7 +1002,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // T_vis sizes the buffers from here on: the exact count of tile visits,
     // or (host-sync-free) an upper bound from the largest support, the
     // kernels reading the exact count on the device.
-    unsigned long long T_vis = 0, num_nonfinite = 0;
+    unsigned long long T_vis = 0, num_nonfinite = 0, visits_bound = 0;
     C->stats.num_points = n_total;
     C->stats_deferred = C->sync_free;
     if (C->sync_free)
@@ -894,8 +1010,8 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         if (before_grid) return fail(MI355_ERR_INVALID_ARG, "host window upload needs host syncs");
         int smax = 0;
         for (size_t p = 0; p < P; ++p) smax = std::max(smax, support[p]);
-        const unsigned long long per = (unsigned long long)(2 * smax / tw + 2) * (2 * smax / th + 2);
-        T_vis = std::max(1ull, n_total * per);
+        visits_bound = (unsigned long long)(2 * smax / tw + 2) * (2 * smax / th + 2);
+        T_vis = std::max(1ull, n_total * visits_bound);
         if (T_vis > 0xFFFFFFFFull)
             return fail(MI355_ERR_TOO_LARGE, "tile-visit bound exceeds 2^32-1 (split the call)");
         num_nonfinite = 1;            // (not known: the pass always runs)
@@ -921,7 +1037,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         if (T_vis == 0)
         {
             record(C, EV_BUCKET); record(C, EV_GRID); record(C, EV_MERGE);
-            TRY(grid_nonfinite<T>(C, num_nonfinite, num_jobs, n_total));
+            TRY(grid_nonfinite<T>(C, num_nonfinite, num_jobs, n_total, lane_cells));
             return commit_jobs<T>(C, num_jobs);
         }
     }
@@ -948,7 +1064,10 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     TRY(radix_sort(C, T_vis, sc + SC_VISITS, key_bits, &cur));
     const unsigned* skeys = C->keys[cur].as<unsigned>();
     // (for mi355_ctx_get_buckets: where this pass's sorted lists are)
-    C->bk_valid = strips && !C->sync_free;
+    C->bk_valid = f32 && (strips || bands) && !C->sync_free;
+    C->bk_bands = bands;
+    C->bk_exact = table_id_shift == 0 && key_table_shift == 0;
+    C->bk_points = n_total;
     C->bk_cur = cur;
     C->bk_count = T_vis;
     C->bk_key_table_bits = key_table_bits;
@@ -960,7 +1079,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // buffers.
     unsigned* run_flag = C->keys[cur ^ 1].as<unsigned>();
     unsigned* run_excl = C->vals[cur ^ 1].as<unsigned>();
-    if (!direct64)
+    if (!direct64 && !bands)
     {
         const int exact_key = table_id_shift == 0 && key_table_shift == 0;
         const unsigned vb = grid_blocks(T_vis, 256, 65535);
@@ -982,13 +1101,24 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
                 strips ? nullptr : C->run_tb.as<int>());
         HIP_TRY(hipGetLastError());
     }
+    if (bands)
+    {
+        TRY(ensure(C, C->vmeta, T_vis * sizeof(int4)));
+        TRY(ensure(C, C->vamp, T_vis * sizeof(T2)));
+        const auto gather = wide ? k_gather_bands<T, double> : k_gather_bands<T, T>;
+        hipLaunchKernelGGL(gather, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0, C->stream,
+                svals, C->vrec.as<VisRec<T>>(), skeys, key_table_bits, C->jobs_d.as<JobDev<T>>(),
+                C->job_tile_base_d.as<unsigned>(), num_jobs, sc + SC_VISITS,
+                C->vmeta.as<int4>(), C->vamp.as<T2>());
+        HIP_TRY(hipGetLastError());
+    }
     if (strips)
     {
         TRY(ensure(C, C->vmeta, T_vis * sizeof(int4)));
         TRY(ensure(C, C->vamp, T_vis * sizeof(T2)));
         TRY(ensure(C, C->vlds, T_vis * sizeof(int)));
         hipLaunchKernelGGL(k_gather_visits<T>, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0,
-                C->stream, svals, C->vrec.as<VisRec>(), run_flag, run_excl,
+                C->stream, svals, C->vrec.as<VisRec<T>>(), run_flag, run_excl,
                 C->run_start.as<unsigned>(), stage_thresholds(C), kStripMaxW, kStripS, skeys,
                 key_table_bits, C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(),
                 num_jobs, th, table_id_shift == 0 ? noff : 0, ov % 2 == 0 ? ov / 2 : -1,
@@ -1008,43 +1138,88 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     hipLaunchKernelGGL(k_fill_u32, dim3(tb), dim3(256), 0, C->stream, C->tile_end.as<unsigned>(), (unsigned long long)num_tiles, 0u);
     hipLaunchKernelGGL(k_tile_bounds, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0, C->stream,
             skeys, sc + SC_VISITS, key_table_bits, C->tile_start.as<unsigned>(), C->tile_end.as<unsigned>());
-    hipLaunchKernelGGL(k_items, dim3(tb), dim3(256), 0, C->stream, C->tile_start.as<unsigned>(),
-            C->tile_end.as<unsigned>(), num_tiles, vpi, C->n_items.as<unsigned>(),
-            C->n_slots.as<unsigned>());
-    HIP_TRY(hipGetLastError());
-    {
+    const size_t slot_bytes = (size_t)(tw * th) * (wide ? sizeof(double2) : sizeof(T2));
+    unsigned long long num_items, num_slots;
+    // items of `override` visits, or of the jobs' own sizes (counts for the
+    // launches: from the device, or, host-sync-free, from bounds)
+    auto make_items = [&](unsigned override) -> int {
+        hipLaunchKernelGGL(k_items<T>, dim3(tb), dim3(256), 0, C->stream,
+                C->tile_start.as<unsigned>(), C->tile_end.as<unsigned>(), num_tiles,
+                C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(), num_jobs, override,
+                C->n_items.as<unsigned>(), C->n_slots.as<unsigned>());
+        HIP_TRY(hipGetLastError());
         DevCount cnt{nullptr, 1, 0, num_tiles};
         TRY(scan_u32(C, C->n_items.as<unsigned>(), C->item_off.as<unsigned>(), cnt, num_tiles,
                 sc + SC_ITEMS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
         TRY(scan_u32(C, C->n_slots.as<unsigned>(), C->slot_off.as<unsigned>(), cnt, num_tiles,
                 sc + SC_SLOTS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
-    }
-    unsigned long long num_items, num_slots;
-    if (C->sync_free)
+        if (C->sync_free)
+        {
+            // a tile of c visits has ceil(c / V) items, and slots only when that
+            // is 2 or more, i.e. fewer than 2c / V
+            num_items = std::min<unsigned long long>(num_tiles, T_vis) + 1;
+            num_slots = 1;
+            for (int j = 0; j < num_jobs; ++j)
+            {
+                const unsigned long long V = override ? override : hj[j].visits_per_item;
+                const unsigned long long c = jobs[j].num_points * visits_bound;
+                num_items += c / V + 1;
+                num_slots += 2 * c / V + 1;
+            }
+        }
+        else
+        {
+            HIP_TRY(hipMemcpyAsync(host_sc, sc, sizeof(host_sc), hipMemcpyDeviceToHost, C->stream));
+            HIP_TRY(hipStreamSynchronize(C->stream));
+            num_items = host_sc[SC_ITEMS];
+            num_slots = host_sc[SC_SLOTS];
+        }
+        return MI355_OK;
+    };
+    // The band kernel takes the jobs' own item sizes, unless one is asked for
+    // or their partial regions would not fit a capped workspace.
+    unsigned override = bands && !C->visits_per_item ? 0u : vpi;
+    TRY(make_items(override));
+    if (!override && !fits(C, C->scratch, num_slots * slot_bytes +
+            num_items * (sizeof(unsigned) + sizeof(BandItem<T>)) + 8192))
     {
-        // a tile of c visits has ceil(c / V) items, and slots only when that
-        // is 2 or more, i.e. fewer than 2c / V
-        const unsigned long long V = vpi;
-        num_items = std::min<unsigned long long>(num_tiles, T_vis) + T_vis / V + 1;
-        num_slots = 2 * T_vis / V + 1;
-    }
-    else
-    {
-        HIP_TRY(hipMemcpyAsync(host_sc, sc, sizeof(host_sc), hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipStreamSynchronize(C->stream));
-        num_items = host_sc[SC_ITEMS];
-        num_slots = host_sc[SC_SLOTS];
+        override = vpi;
+        TRY(make_items(override));
     }
     TRY(ensure(C, C->item_tile, num_items * sizeof(unsigned)));
     hipLaunchKernelGGL(k_item_map, dim3(tb), dim3(256), 0, C->stream, C->item_off.as<unsigned>(),
             num_tiles, C->item_tile.as<unsigned>());
     HIP_TRY(hipGetLastError());
+    if (bands)
+    {
+        // in table order where that pays (larger calls)
+        const bool ordered = n_total >= kBandOrderMin;
+        TRY(ensure(C, C->band_items, num_items * sizeof(BandItem<T>)));
+        TRY(ensure(C, C->order_count, kOrderBuckets * sizeof(unsigned)));
+        unsigned* first = ordered ? C->order_count.as<unsigned>() : nullptr;
+        BandItemArgs ba{C->item_off.as<unsigned>() + num_tiles, C->item_tile.as<unsigned>(),
+                C->item_off.as<unsigned>(), C->slot_off.as<unsigned>(), C->tile_start.as<unsigned>(),
+                C->tile_end.as<unsigned>(), skeys, override, (unsigned)((1ull << key_table_bits) - 1),
+                std::max(0, key_table_bits - bits_for(kOrderBuckets)),
+                C->job_tile_base_d.as<unsigned>(), num_jobs, tw, th};
+        const dim3 ib(grid_blocks(num_items, 256, 1024));
+        if (ordered)
+        {
+            hipLaunchKernelGGL(k_fill_u32, dim3(4), dim3(256), 0, C->stream, first,
+                    (unsigned long long)kOrderBuckets, 0u);
+            hipLaunchKernelGGL(k_order_count<T>, ib, dim3(256), 0, C->stream, ba,
+                    C->jobs_d.as<JobDev<T>>(), first);
+            hipLaunchKernelGGL(k_order_scan, dim3(1), dim3(kOrderBuckets), 0, C->stream, first);
+        }
+        hipLaunchKernelGGL(k_band_items<T>, ib, dim3(256), 0, C->stream, ba,
+                C->jobs_d.as<JobDev<T>>(), first, C->band_items.as<BandItem<T>>());
+        HIP_TRY(hipGetLastError());
+    }
     record(C, EV_BUCKET);
     C->stats.num_items = num_items;
 
     // Grid.
-    const size_t part_bytes = comp ? sizeof(double2) : sizeof(T2);
-    TRY(ensure(C, C->scratch, num_slots * (unsigned long long)(tw * th) * part_bytes));
+    TRY(ensure(C, C->scratch, num_slots * slot_bytes));
     GridArgs<T> ga;
     ga.tables = C->tables.as<T2>();
     ga.table_bytes = (unsigned)((C->table_elems + C->table_tail) * sizeof(T2));
@@ -1071,12 +1246,13 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     ga.d_num_runs = sc + SC_RUNS;
     ga.min_stage_run = C->min_stage_run ? C->min_stage_run
                                         : stage_run_default(std::is_same<T, double>::value);
-    if (strips && (T_vis + 1) * 4ull > 0xFFFFFFFFull)
+    if ((strips || bands) && (T_vis + 1) * 4ull > 0xFFFFFFFFull)
         return fail(MI355_ERR_TOO_LARGE, "more than 2^30 tile visits in one call");
     ga.vmeta = C->vmeta.as<int4>();
     ga.vamp = C->vamp.as<T2>();
     ga.vlds = C->vlds.as<int>();
     ga.item_group = C->item_group;
+    ga.band_items = C->band_items.as<BandItem<T>>();
     // the strip kernel's persistent grid takes positions from per-XCD
     // counters (zeroed with the other scalars at the start of the pass)
     ga.item_ctr = reinterpret_cast<unsigned*>(sc + SC_ITEM_CTR);
@@ -1090,7 +1266,19 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     const unsigned wg_items = C->sync_free
             ? (unsigned)std::min<unsigned long long>(num_items, 2ull * C->num_cu)
             : (unsigned)num_items;
-    if (num_items && strips)
+    if (num_items && bands)
+    {
+        // one workgroup (one wave) per share of an item, in whole eights;
+        // host-sync-free, where num_items is a bound, at most 2^17
+        const unsigned long long blk = 8ull * C->item_group;
+        unsigned long long wg = (num_items + blk - 1) / blk * blk * BandPlain::kWork;
+        if (C->sync_free) wg = std::min(wg, 1ull << 17);
+        if (wg > 0x7FFFFFFFull / 64) wg = 0x7FFFFFFFull / 64 & ~7ull;
+        const auto kernel = wide ? k_grid_bands<T, double> : k_grid_bands<T, T>;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3(64), 0, C->stream, ga);
+        HIP_TRY(hipGetLastError());
+    }
+    else if (num_items && strips)
     {
         if constexpr (std::is_same<T, float>::value)
         {
@@ -1154,7 +1342,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         HIP_TRY(hipGetLastError());
     }
     record(C, EV_MERGE);
-    TRY(grid_nonfinite<T>(C, num_nonfinite, num_jobs, n_total));
+    TRY(grid_nonfinite<T>(C, num_nonfinite, num_jobs, n_total, lane_cells));
     return commit_jobs<T>(C, num_jobs);
 }
 
@@ -1416,7 +1604,7 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     HIP_TRY(hipSetDevice(C->device));
     typedef typename V2<T>::t T2;
     typedef typename V4<T>::t T4;
-    TRY((prepare_tables<T, T>(C, P, support, ov, csh, reinterpret_cast<const T2*>(conv))));
+    TRY((prepare_tables<T, T>(C, P, support, ov, csh, reinterpret_cast<const T2*>(conv), 0)));
     const int half = (ov + 1) / 2, noff = half + 1;
     // One job; its norm/skipped totals go to library scratch (not reported).
     TRY(ensure(C, C->in_norm, sizeof(double)));
@@ -2065,8 +2253,33 @@ MI355_EXPORT int mi355_ctx_get_buckets(mi355_ctx* C, unsigned long long* count,
                 C->stream));
     }
     HIP_TRY(hipStreamSynchronize(C->stream));
-    for (size_t i = 0; i < vm.size(); ++i)
-        flags[i] = ((vm[i].z & kVisitStaged) ? 1 : 0) | ((vm[i].z & kVisitRunStart) ? 2 : 0);
+    if (!C->bk_bands)
+    {
+        for (size_t i = 0; i < vm.size(); ++i)
+            flags[i] = ((vm[i].z & kVisitStaged) ? 1 : 0) | ((vm[i].z & kVisitRunStart) ? 2 : 0);
+        return ok();
+    }
+    // The band kernel has no runs: what the strip kernel would make of the
+    // same lists (table widths in the band records).
+    std::vector<unsigned> hk(vm.size()), hv(vm.size());
+    std::vector<int4> hm;
+    HIP_TRY(hipMemcpy(hk.data(), C->keys[C->bk_cur].p, vm.size() * sizeof(unsigned), hipMemcpyDeviceToHost));
+    if (!C->bk_exact && !vm.empty())
+    {
+        hm.resize((size_t)C->bk_points);
+        HIP_TRY(hipMemcpy(hv.data(), C->vals[C->bk_cur].p, vm.size() * sizeof(unsigned), hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(hm.data(), C->meta.p, hm.size() * sizeof(int4), hipMemcpyDeviceToHost));
+    }
+    const uint4 thr = stage_thresholds(C);
+    for (size_t i = 0, e; i < vm.size(); i = e)
+    {
+        for (e = i + 1; e < vm.size() && hk[e] == hk[i] &&
+                (C->bk_exact || hm[hv[e]].w == hm[hv[i]].w); ++e) { }
+        const int W = vm[i].w & 0xffff;
+        const unsigned need = W <= 33 ? thr.x : W <= 65 ? thr.y : W <= 97 ? thr.z : thr.w;
+        for (size_t q = i; q < e; ++q)
+            flags[q] = (e - i >= need && W <= kStripMaxW ? 1 : 0) | (q == i ? 2 : 0);
+    }
     return ok();
 }
 
@@ -2407,25 +2620,30 @@ MI355_EXPORT int mi355_autotune_f_batched_dev(mi355_ctx* C, size_t P, const int*
     st = trial(t);
     // Stage 1: kernel / geometry, work-item size, item grouping, with one
     // staged-run threshold for every class.
+    // A threshold of 0 is the automatic kernel, tried first where that is the
+    // band kernel (which has item sizes of its own).
     const unsigned zero4[4] = {0, 0, 0, 0};
+    auto stage1 = [&](int kern, unsigned vpi, unsigned msr, unsigned grp) {
+        if (st != MI355_OK) return;
+        apply(kern, vpi, msr, grp, zero4);
+        st = trial(t);
+        if (st == MI355_OK && t < best_t)
+        {
+            best_t = t;
+            best = Setting{kern, vpi, msr, grp, {0, 0, 0, 0}};
+        }
+    };
+    apply(0, 0, 0, 1, zero4);
+    if (st == MI355_OK && auto_kernel_is_bands(C, P, support, ov, num_jobs, J.data()))
+        for (unsigned vpi : {0u, 1024u, 2048u, 4096u}) stage1(0, vpi, 0u, 1u);
     for (int kern : {0, 2})
         for (unsigned vpi : {1024u, 2048u, 4096u, 8192u})
             for (unsigned grp : {1u, 8u})
-            {
-                if (st != MI355_OK) break;
-                if (kern == 2 && grp != 1u) continue;
-                apply(kern, vpi, kern == 2 ? 4u : 3u, grp, zero4);
-                st = trial(t);
-                if (st == MI355_OK && t < best_t)
-                {
-                    best_t = t;
-                    best = Setting{kern, vpi, C->min_stage_run, grp, {0, 0, 0, 0}};
-                }
-            }
+                if (kern == 0 || grp == 1u) stage1(kern, vpi, kern == 2 ? 4u : 3u, grp);
     // Stage 2 (strip kernel): each support class's threshold in turn, the
     // others held at their best so far; two passes per value, the faster
     // counts.
-    if (st == MI355_OK && best.kernel == 0)
+    if (st == MI355_OK && best.kernel == 0 && best.msr != 0)
     {
         for (int c = 0; c < 4 && st == MI355_OK; ++c)
         {

@@ -103,9 +103,14 @@ MI355_EXPORT int mi355_ctx_get_stream(mi355_ctx* ctx, void** hip_stream);
 #define MI355_OPT_PHASE_TIMING    3  /* 1: record hipEvents around each phase */
 #define MI355_OPT_CACHE_KERNELS   4  /* 1: reuse prepared kernel tables while the
                                         conv_func pointer and shape are unchanged */
-#define MI355_OPT_GRID_KERNEL     5  /* 0: automatic (default): 16-column strips on
-                                        256x128 regions for FP32 (192x64 when
-                                        compensated), 2 for FP64;
+#define MI355_OPT_GRID_KERNEL     5  /* 0: automatic (default): for FP64 the band
+                                        kernel (8-row bands with the cells in LDS);
+                                        for FP32 and compensated FP32 the band
+                                        kernel where tables serve few visits, else
+                                        16-column strips on 256x128 regions (192x64
+                                        when compensated).  With a staged-run
+                                        threshold set (below): strips for FP32, 2
+                                        for FP64;
                                         1: 64x64 tiles, tables read directly;
                                         2: 64x64 tiles, tables staged in LDS */
 #define MI355_OPT_MIN_STAGE_RUN   6  /* shortest same-table run staged in LDS;
@@ -150,21 +155,24 @@ typedef struct
     unsigned long long num_taps;    /* sum over gridded visibilities of (2s+1)^2 */
     unsigned long long num_merge_tiles;
     unsigned long long visits_per_item;  /* work-item size used (the option, or
-                                            the automatic choice) */
+                                            the automatic choice; the band kernel
+                                            splits automatic items further) */
 } mi355_stats;
 
 MI355_EXPORT int mi355_ctx_get_stats(const mi355_ctx* ctx, mi355_stats* stats);
 
-/* Introspection of the last FP32 strip-kernel gridding pass on the context
- * (not a host-synchronisation-free one): its sorted tile lists, for checking
+/* Introspection of the last FP32 strip- or band-kernel gridding pass on the
+ * context (not a host-synchronisation-free or, on the band kernel, a
+ * compensated one, whose regions are smaller): its sorted tile lists, for checking
  * the bucketing against a restatement of the selection.  *count receives
  * the number of (region, visibility) visits and *key_table_bits the number
  * of low key bits below the region id; with cap >= *count, keys[i] and
  * vis[i] receive the i-th sorted visit's key ((region << key_table_bits) |
  * kernel-table id) and visibility index, and flags[i] bit 0 = the visit's
- * run is staged in LDS, bit 1 = the visit starts a run (any output may be
- * NULL).  No reference counterpart: it stands for the per-tile count and
- * scatter of oskar_grid_wproj_gpu.cu:359-649. */
+ * run is staged in LDS by the strip kernel (after a band-kernel pass: would
+ * be), bit 1 = the visit starts a run (any output may be NULL).  No
+ * reference counterpart: it stands for the per-tile count and scatter of
+ * oskar_grid_wproj_gpu.cu:359-649. */
 MI355_EXPORT int mi355_ctx_get_buckets(mi355_ctx* ctx, unsigned long long* count,
         int* key_table_bits, unsigned* keys, unsigned* vis, int* flags, unsigned long long cap);
 
@@ -307,9 +315,9 @@ MI355_EXPORT int mi355_grid_wproj_f_batched_graph_dev(mi355_ctx* ctx,
 
 /* Autotuner for a batched workload: times the pipeline into private
  * outputs (one scratch grid per job; the job table's grids are not
- * touched), first over the gridding kernel / tile geometry (16-column
- * strips on 256x128 regions, or 64x64 tiles), work-item size and item
- * grouping, then, for the strip kernel, over the shortest staged run of
+ * touched), first over the gridding kernel / tile geometry (the band
+ * kernel where that is the automatic one, 16-column strips on 256x128
+ * regions, or 64x64 tiles), work-item size and item grouping, then, for the strip kernel, over the shortest staged run of
  * each support class in turn (tables at most 33, 65, 97, 111 wide), and
  * leaves the fastest settings in the context's options
  * (MI355_OPT_GRID_KERNEL, _VISITS_PER_ITEM, _ITEM_GROUP, _MIN_STAGE_RUN,
