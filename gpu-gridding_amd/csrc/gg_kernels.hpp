@@ -1291,15 +1291,25 @@ void k_grid_nonfinite(const typename V2<T>::t* __restrict__ tables,
 // ===========================================================================
 // Degridding (adjoint)
 // ===========================================================================
-// One wave per visibility.  The footprint's W*W taps are dealt to the 64
-// lanes in row-major order (lane l takes taps l, l+64, ...: row t / W,
-// column t % W, kept up incrementally), so every lane works whatever W is
-// and a wave's 64 table reads are one contiguous run; per-lane partials are
-// reduced across the wave at the end.  The visibilities go in the order
-// `order` gives (grid tiles of their centre cells: waves that run together
-// read neighbouring cells), or in index order when it is null.  Output per
-// visibility: sum over taps of conj-folded tap * grid cell, times the
-// weight when apply_weight (the adjoint of oskar_grid_wproj.c:190-209).
+// One wave per visibility, its footprint walked in units of 8 rows x 8 lanes:
+// a lane takes 16 bytes of the table and of the grid at a time (two adjacent
+// complex FP32 values, or one FP64 one), the units of 8 rows side by side in
+// one straight-line block, so that every address but the first is an
+// immediate and a block's loads are in flight together.  What binds it is the
+// vector load path (16 bytes per FP32 tap; 41 of its 64 bytes per clock and
+// CU are moved, 1M visibilities of support up to 32 on a 4096^2 grid: 1.44 ms
+// with one tap and one cell of 8 bytes per lane and load, 1.25 ms so; blocks
+// of at most 4 or 5 units, which leave registers for twice the waves, 1.33 and
+// 1.29 ms).  Lanes past the
+// footprint read nothing (out of the buffers' range: zeros) and the half of a
+// pair that lies past its last column is masked, so cells outside the
+// footprint (which may hold anything) never reach a sum.  The visibilities go
+// in the order `order` gives (grid tiles of their centre cells: waves that run
+// together read neighbouring cells), or in index order when it is null.
+// Output per visibility: sum over taps of conj-folded tap * grid cell, times
+// the weight when apply_weight (the adjoint of oskar_grid_wproj.c:190-209).
+constexpr unsigned kOutOfRange = 0x80000000u;
+
 template <typename T>
 __global__ __launch_bounds__(256)
 void k_degrid(const typename V2<T>::t* __restrict__ tables,
@@ -1309,7 +1319,14 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
         typename V2<T>::t* __restrict__ out)
 {
     typedef typename V2<T>::t T2;
+    constexpr int LC = sizeof(T) == 4 ? 2 : 1;           // values per lane
+    constexpr int kUnit = 8 * LC;                        // columns of a unit
+    constexpr int kMaxUnits = sizeof(T) == 4 ? 8 : 4;    // units of one block
+    constexpr int kSize = (int)sizeof(T2);
+    struct Vals { T v[2 * LC]; };
     const int lane = lane_id();
+    const int lr = lane >> 3, lc = lane & 7;
+    const unsigned row_bytes = (unsigned)grid_size * kSize;
     const unsigned long long nw = (unsigned long long)gridDim.x * (blockDim.x >> 6);
     const unsigned long long w0 = (unsigned long long)blockIdx.x * (blockDim.x >> 6) +
             (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1317,40 +1334,100 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
     {
         const unsigned long long i = order ? (unsigned long long)ld_const(order, q) : q;
         const int4 mt = ld_const(meta, i);
-        T re = (T)0, im = (T)0;
+        T re[LC], im[LC];
+        #pragma unroll
+        for (int h = 0; h < LC; ++h) re[h] = im[h] = (T)0;
         if (!(mt.z & kFlagSkip))
         {
             const int s = meta_support(mt.z);
             const int W = 2 * s + 1;
-            const int n2 = W * W;
-            const bool neg_u = mt.z & kFlagNegU, neg_v = mt.z & kFlagNegV;
+            const bool nv = mt.z & kFlagNegV;
             const T cj = (mt.z & kFlagConj) ? (T)-1 : (T)1;
-            // 64 taps further on: dr rows and dc columns (one more row when
-            // the column passes W)
-            const int dr = 64 / W, dc = 64 - dr * W;
-            int r = lane / W, c = lane - (lane / W) * W;
             const T2* tab = tables + (unsigned)mt.w;                 // table row 0
             const T2* g0 = grid + (size_t)(mt.y - s) * grid_size + (mt.x - s);
-            for (int t = lane; t < n2; t += 64)
-            {
-                const int tr = neg_v ? W - 1 - r : r;
-                const int tc = neg_u ? W - 1 - c : c;
-                const T2 cv = tab[tr * W + tc];
-                const T2 g = g0[r * grid_size + c];
-                const T ci = cv.y * cj;
-                re = fma(cv.x, g.x, re); re = fma(ci, g.y, re);
-                im = fma(cv.x, g.y, im); im = fma(-ci, g.x, im);
-                r += dr;
-                c += dc;
-                if (c >= W) { c -= W; ++r; }
-            }
+            // Columns c0 .. of the footprint, N units wide (the last one may
+            // be cut off by the footprint's edge), all its rows.
+            auto columns = [&](int c0, auto mirrored, auto units) {
+                constexpr bool MIR = decltype(mirrored)::value;
+                constexpr int N = decltype(units)::value;
+                // the lane's offsets in a block of 8 rows; table blocks and
+                // columns that run backwards are addressed from their low end
+                const unsigned to = (unsigned)((nv ? 7 - lr : lr) * W + (MIR ? 7 - lc : lc) * LC) * kSize;
+                const unsigned go = (unsigned)lr * row_bytes + (unsigned)(lc * LC * kSize);
+                const int tc = MIR ? W - c0 - N * kUnit : c0;
+                const T2* tp = tab + (nv ? W - 8 : 0) * W + tc;
+                const T2* gp = g0 + c0;
+                const int last = c0 + (N - 1) * kUnit + lc * LC;     // column in the last unit
+                for (int r0 = 0; r0 < W; r0 += 8)
+                {
+                    const __amdgpu_buffer_rsrc_t rt = table_rsrc(tp, 0x7fffffffu);
+                    const __amdgpu_buffer_rsrc_t rg = table_rsrc(gp, 0x7fffffffu);
+                    const bool row = r0 + lr < W, end = row && last < W;
+                    const unsigned t0 = row ? to : kOutOfRange, g1 = row ? go : kOutOfRange;
+                    const unsigned tl = end ? to : kOutOfRange, gl = end ? go : kOutOfRange;
+                    Vals c[N], g[N];
+                    #pragma unroll
+                    for (int u = 0; u < N; ++u)
+                    {
+                        const bool e = u == N - 1;
+                        c[u] = __builtin_bit_cast(Vals, __builtin_amdgcn_raw_buffer_load_b128(rt,
+                                (int)(e ? tl : t0) + (MIR ? N - 1 - u : u) * kUnit * kSize, 0, 0));
+                        g[u] = __builtin_bit_cast(Vals, __builtin_amdgcn_raw_buffer_load_b128(rg,
+                                (int)(e ? gl : g1) + u * kUnit * kSize, 0, 0));
+                    }
+                    #pragma unroll
+                    for (int u = 0; u < N; ++u)
+                    {
+                        #pragma unroll
+                        for (int h = 0; h < LC; ++h)
+                        {
+                            const int hk = MIR ? LC - 1 - h : h;
+                            T cx = c[u].v[2 * hk], ci = c[u].v[2 * hk + 1] * cj;
+                            T gx = g[u].v[2 * h], gy = g[u].v[2 * h + 1];
+                            if (h > 0 && u == N - 1)
+                            {
+                                const bool in = last + h < W;
+                                cx = in ? cx : (T)0; ci = in ? ci : (T)0;
+                                gx = in ? gx : (T)0; gy = in ? gy : (T)0;
+                            }
+                            re[h] = fma(cx, gx, re[h]); re[h] = fma(ci, gy, re[h]);
+                            im[h] = fma(cx, gy, im[h]); im[h] = fma(-ci, gx, im[h]);
+                        }
+                    }
+                    tp += (nv ? -8 : 8) * W;
+                    gp += (size_t)8 * grid_size;
+                }
+            };
+            auto footprint = [&](auto mirrored) {
+                int c0 = 0;
+                for (; W - c0 > kMaxUnits * kUnit; c0 += kMaxUnits * kUnit)
+                    columns(c0, mirrored, std::integral_constant<int, kMaxUnits>());
+                const int units = (W - c0 + kUnit - 1) / kUnit;
+                if constexpr (kMaxUnits == 8)
+                    switch (units)
+                    {
+                    case 4: columns(c0, mirrored, std::integral_constant<int, 4>()); return;
+                    case 5: columns(c0, mirrored, std::integral_constant<int, 5>()); return;
+                    case 6: columns(c0, mirrored, std::integral_constant<int, 6>()); return;
+                    case 7: columns(c0, mirrored, std::integral_constant<int, 7>()); return;
+                    }
+                switch (units)
+                {
+                case 1: columns(c0, mirrored, std::integral_constant<int, 1>()); return;
+                case 2: columns(c0, mirrored, std::integral_constant<int, 2>()); return;
+                case 3: columns(c0, mirrored, std::integral_constant<int, 3>()); return;
+                default: columns(c0, mirrored, std::integral_constant<int, kMaxUnits>()); return;
+                }
+            };
+            if (mt.z & kFlagNegU) footprint(std::true_type());
+            else footprint(std::false_type());
         }
-        re = wave_sum(re);
-        im = wave_sum(im);
+        if (LC == 2) { re[0] += re[LC - 1]; im[0] += im[LC - 1]; }
+        const T sr = wave_sum(re[0]), si = wave_sum(im[0]);
         if (lane == 0)
         {
             const T w = apply_weight ? weight[i] : (T)1;
-            T2 v; v.x = re * w; v.y = im * w;
+            T2 v; v.x = sr * w; v.y = si * w;
             out[i] = v;
         }
     }
