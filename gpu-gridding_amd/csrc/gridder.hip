@@ -1970,32 +1970,46 @@ int image_dev(mi355_ctx* C, int G, const T* grid, double norm, T* image)
     HIP_TRY(hipSetDevice(C->device));
     typedef typename V2<T>::t T2;
     const unsigned long long n = (unsigned long long)G * G;
-    TRY(ensure(C, C->fft_work, n * sizeof(T2)));
+    const size_t half_bytes = (size_t)G * (G / 2 + 1) * sizeof(T2);    // the half spectrum
+    // The transform writes the image unless its pointer is less aligned than
+    // the transform's wide stores may assume.
+    const bool direct = ((uintptr_t)image & 15u) == 0;
+    const size_t tmp_at = (half_bytes + 255) & ~(size_t)255;
+    TRY(ensure(C, C->fft_work, direct ? half_bytes : tmp_at + n * sizeof(T)));
+    T* real = direct ? image : reinterpret_cast<T*>(C->fft_work.as<unsigned char>() + tmp_at);
     const int dbl = sizeof(T) == 8;
     if (!C->fft_valid || C->fft_G != G || C->fft_double != dbl)
     {
         if (C->fft_valid) (void)hipfftDestroy(C->fft_plan);
         C->fft_valid = false;
-        FFT_TRY(hipfftPlan2d(&C->fft_plan, G, G, dbl ? HIPFFT_Z2Z : HIPFFT_C2C));
+        FFT_TRY(hipfftPlan2d(&C->fft_plan, G, G, dbl ? HIPFFT_Z2D : HIPFFT_C2R));
         C->fft_valid = true;
         C->fft_G = G;
         C->fft_double = dbl;
     }
     FFT_TRY(hipfftSetStream(C->fft_plan, C->stream));
-    const unsigned blocks = grid_blocks(n / 2, 256, 65535);
-    hipLaunchKernelGGL(k_image_pre<T>, dim3(blocks), dim3(256), 0, C->stream,
-            reinterpret_cast<const T2*>(grid), C->fft_work.as<T2>(), (unsigned)G, n / 2);
+    // The scale goes in before the transform where it cannot push values out
+    // of range, after it otherwise.
+    const T scale = (T)(norm != 0.0 ? 1.0 / norm : 1.0);
+    const T mag = scale < (T)0 ? -scale : scale;
+    const bool early = direct && mag > (T)1e-15 && mag < (T)1e15;
+    const dim3 pre(grid_blocks(G / 2 + 1, 256, 256), (unsigned)std::min(G, 65535));
+    hipLaunchKernelGGL(k_image_pre<T>, pre, dim3(256), 0, C->stream,
+            reinterpret_cast<const T2*>(grid), C->fft_work.as<T2>(), (unsigned)G,
+            (T)0.5 * (early ? scale : (T)1));
     HIP_TRY(hipGetLastError());
     if (dbl)
-        FFT_TRY(hipfftExecZ2Z(C->fft_plan, C->fft_work.as<hipfftDoubleComplex>(),
-                C->fft_work.as<hipfftDoubleComplex>(), HIPFFT_BACKWARD));
+        FFT_TRY(hipfftExecZ2D(C->fft_plan, C->fft_work.as<hipfftDoubleComplex>(),
+                reinterpret_cast<hipfftDoubleReal*>(real)));
     else
-        FFT_TRY(hipfftExecC2C(C->fft_plan, C->fft_work.as<hipfftComplex>(),
-                C->fft_work.as<hipfftComplex>(), HIPFFT_BACKWARD));
-    const T scale = (T)(norm != 0.0 ? 1.0 / norm : 1.0);
-    hipLaunchKernelGGL(k_image_post<T>, dim3(blocks), dim3(256), 0, C->stream,
-            C->fft_work.as<T2>(), image, (unsigned)G, n / 2, scale);
-    HIP_TRY(hipGetLastError());
+        FFT_TRY(hipfftExecC2R(C->fft_plan, C->fft_work.as<hipfftComplex>(),
+                reinterpret_cast<hipfftReal*>(real)));
+    if (!early)
+    {
+        hipLaunchKernelGGL(k_image_scale<T>, dim3(grid_blocks(n, 1024, 65535)), dim3(256), 0,
+                C->stream, real, image, n, scale);
+        HIP_TRY(hipGetLastError());
+    }
     return ok();
 }
 

@@ -399,10 +399,11 @@ MI355_EXPORT int mi355_grid_weights_read_d_dev(mi355_ctx* ctx, size_t num_points
  * (1/norm taken as 1 when norm is 0): the centred inverse transform, so a
  * grid holding one value at cell (c, c) gives a constant image.  grid is G*G
  * complex values (interleaved re, im, row-major), image G*G reals.  hipFFT
- * does the transform; two HIP passes apply the centring signs and the
- * scale.  Odd grid sizes: MI355_ERR_INVALID_ARG; above 65536:
- * MI355_ERR_TOO_LARGE.  The device forms use a work buffer of G*G complex
- * values kept in the context.
+ * does the transform (complex to real, of the input's Hermitian part, which
+ * a HIP pass forms with the centring signs and the scale).  Odd grid sizes:
+ * MI355_ERR_INVALID_ARG; above 65536: MI355_ERR_TOO_LARGE.  The device forms
+ * use a work buffer of G*(G/2+1) complex values kept in the context (and G*G
+ * reals more for an image that is not 16-byte aligned).
  * ---------------------------------------------------------------------- */
 MI355_EXPORT void mi355_grid_to_image_f(int grid_size, const float* grid, double norm,
         float* image);
