@@ -78,19 +78,6 @@ struct BandItem
     typename V2<T>::t* grid;
 };
 
-__device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
-__device__ __forceinline__ float read_lane(float v, int l)
-{
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
-}
-__device__ __forceinline__ double read_lane(double v, int l)
-{
-    const long long b = __builtin_bit_cast(long long, v);
-    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)b, l);
-    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 template <typename TAP, typename CELL>
 __global__ __launch_bounds__(64)
 void k_grid_bands(const GridArgs<TAP> A)

@@ -462,6 +462,25 @@ __device__ __forceinline__ unsigned long long block_excl_scan_u64(
     return base + v - x;
 }
 
+// One thread's elements (zeros past the end), 16 bytes a load: `in` is the
+// start of an allocation and base a multiple of 16.
+__device__ __forceinline__ void scan_load(const unsigned* __restrict__ in,
+        unsigned long long base, unsigned long long n, unsigned (&vals)[kScanPerThread])
+{
+    if (base + kScanPerThread <= n)
+    {
+        #pragma unroll
+        for (int q = 0; q < kScanPerThread; q += 4)
+        {
+            const uint4 x = *reinterpret_cast<const uint4*>(in + base + q);
+            vals[q] = x.x; vals[q + 1] = x.y; vals[q + 2] = x.z; vals[q + 3] = x.w;
+        }
+        return;
+    }
+    #pragma unroll
+    for (int q = 0; q < kScanPerThread; ++q) vals[q] = base + q < n ? in[base + q] : 0u;
+}
+
 __global__ __launch_bounds__(kScanThreads)
 void k_scan_reduce(const unsigned* __restrict__ in, DevCount cnt,
         unsigned long long* __restrict__ partial)
@@ -472,10 +491,11 @@ void k_scan_reduce(const unsigned* __restrict__ in, DevCount cnt,
     for (unsigned long long c = blockIdx.x; c < nchunk; c += gridDim.x)
     {
         const unsigned long long base = c * kScanChunk + (unsigned long long)threadIdx.x * kScanPerThread;
+        unsigned vals[kScanPerThread];
+        scan_load(in, base, n, vals);
         unsigned long long s = 0;
         #pragma unroll
-        for (int q = 0; q < kScanPerThread; ++q)
-            if (base + q < n) s += in[base + q];
+        for (int q = 0; q < kScanPerThread; ++q) s += vals[q];
         unsigned long long tot;
         block_excl_scan_u64(s, sh, &tot);
         if (threadIdx.x == 0) partial[c] = tot;
@@ -535,20 +555,30 @@ void k_scan_down(const unsigned* __restrict__ in, DevCount cnt,
     {
         const unsigned long long base = c * kScanChunk + (unsigned long long)threadIdx.x * kScanPerThread;
         unsigned vals[kScanPerThread];
+        scan_load(in, base, n, vals);
         unsigned long long s = 0;
         #pragma unroll
-        for (int q = 0; q < kScanPerThread; ++q)
-        {
-            vals[q] = base + q < n ? in[base + q] : 0u;
-            s += vals[q];
-        }
+        for (int q = 0; q < kScanPerThread; ++q) s += vals[q];
         unsigned long long tot;
         unsigned long long run = partial[c] + block_excl_scan_u64(s, sh, &tot);
         #pragma unroll
         for (int q = 0; q < kScanPerThread; ++q)
         {
-            if (base + q < n) out[base + q] = (unsigned)run;
-            run += vals[q];
+            const unsigned x = vals[q];
+            vals[q] = (unsigned)run;
+            run += x;
+        }
+        if (base + kScanPerThread <= n)
+        {
+            #pragma unroll
+            for (int q = 0; q < kScanPerThread; q += 4)
+                *reinterpret_cast<uint4*>(out + base + q) =
+                        make_uint4(vals[q], vals[q + 1], vals[q + 2], vals[q + 3]);
+        }
+        else
+        {
+            #pragma unroll
+            for (int q = 0; q < kScanPerThread; ++q) if (base + q < n) out[base + q] = vals[q];
         }
     }
 }
@@ -600,9 +630,12 @@ void k_emit(const int4* __restrict__ meta, const unsigned* __restrict__ num_visi
 constexpr int kSortThreads = 256;
 constexpr int kSortPerThread = 16;
 constexpr int kSortChunk = kSortThreads * kSortPerThread;
+constexpr int kScatterThreads = 512;
 
 // Histogram of one BITS-bit digit (8 or 9) per chunk, stored digit-major:
-// hist[d * nchunk + c].
+// hist[d * nchunk + c].  Counts go to four copies in neighbouring banks, lane
+// modulo 4: keys in runs (the later passes' input) would add to one address
+// from a whole wave.  With 16-byte loads, 31.4M keys: 67 -> 41 us a pass.
 template <int BITS>
 __global__ __launch_bounds__(kSortThreads)
 void k_sort_hist(const unsigned* __restrict__ keys,
@@ -611,22 +644,41 @@ void k_sort_hist(const unsigned* __restrict__ keys,
 {
     constexpr int R = 1 << BITS;
     constexpr unsigned M = R - 1;
-    __shared__ unsigned h[R];
+    constexpr int kCopies = 4;
+    __shared__ unsigned h[R * kCopies];
     const unsigned long long n = *d_n;
     const unsigned long long nchunk = (n + kSortChunk - 1) / kSortChunk;
     for (unsigned long long c = blockIdx.x; c < nchunk; c += gridDim.x)
     {
-        for (int d = threadIdx.x; d < R; d += kSortThreads) h[d] = 0;
+        for (int d = threadIdx.x; d < R * kCopies; d += kSortThreads) h[d] = 0;
         __syncthreads();
-        const unsigned long long base = c * kSortChunk;
-        #pragma unroll 4
-        for (int r = 0; r < kSortPerThread; ++r)
+        const unsigned long long base = c * kSortChunk + threadIdx.x * 4;
+        unsigned* mine = h + (threadIdx.x & (kCopies - 1));
+        uint4 k[kSortPerThread / 4];
+        #pragma unroll
+        for (int r = 0; r < kSortPerThread / 4; ++r)
         {
-            const unsigned long long idx = base + r * kSortThreads + threadIdx.x;
-            if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & M], 1u);
+            const unsigned long long idx = base + r * (kSortThreads * 4);
+            if (idx + 4 <= n) k[r] = *reinterpret_cast<const uint4*>(keys + idx);
+        }
+        #pragma unroll
+        for (int r = 0; r < kSortPerThread / 4; ++r)
+        {
+            const unsigned long long idx = base + r * (kSortThreads * 4);
+            if (idx + 4 <= n)
+            {
+                atomicAdd(&mine[((k[r].x >> shift) & M) * kCopies], 1u);
+                atomicAdd(&mine[((k[r].y >> shift) & M) * kCopies], 1u);
+                atomicAdd(&mine[((k[r].z >> shift) & M) * kCopies], 1u);
+                atomicAdd(&mine[((k[r].w >> shift) & M) * kCopies], 1u);
+            }
+            else
+                for (unsigned long long i = idx; i < n; ++i)
+                    atomicAdd(&mine[((keys[i] >> shift) & M) * kCopies], 1u);
         }
         __syncthreads();
-        for (int d = threadIdx.x; d < R; d += kSortThreads) hist[d * nchunk + c] = h[d];
+        for (int d = threadIdx.x; d < R; d += kSortThreads)
+            hist[d * nchunk + c] = h[d * 4] + h[d * 4 + 1] + h[d * 4 + 2] + h[d * 4 + 3];
         __syncthreads();
     }
 }
@@ -638,22 +690,28 @@ void k_sort_hist(const unsigned* __restrict__ keys,
 // lowest lane of each digit group advances it).  One prefix over the waves
 // per digit then gives each wave's base, so that ranks follow index order
 // and the chunk's base for each digit comes from the digit-major scan.  The
-// keys, values and ranks stay in registers meanwhile: two barriers per
-// chunk.
-template <int BITS>
-__global__ __launch_bounds__(kSortThreads)
+// pairs are then put in their chunk's sorted order in LDS and stored from
+// there: neighbouring lanes write neighbouring addresses of one digit's run,
+// where stores straight from the registers went to up to 64 lines each
+// (31.4M pairs, one pass of 8 bits: 239 -> 164 us, 3.1 TB/s; chunks of 2048
+// 190, of 8192 204; 256 threads 167, 1024 227).
+template <int BITS, typename V>
+__global__ __launch_bounds__(kScatterThreads)
 void k_sort_scatter(const unsigned* __restrict__ keys_in,
-        const unsigned* __restrict__ vals_in,
+        const V* __restrict__ vals_in,
         const unsigned long long* __restrict__ d_n, int shift,
         const unsigned* __restrict__ hist_off,
-        unsigned* __restrict__ keys_out, unsigned* __restrict__ vals_out)
+        unsigned* __restrict__ keys_out, V* __restrict__ vals_out)
 {
     constexpr int R = 1 << BITS;
     constexpr unsigned M = R - 1;
-    constexpr int NW = kSortThreads / 64;
+    constexpr int NW = kScatterThreads / 64;
     constexpr int SUB = kSortChunk / NW / 64;          // 64-element rows per wave
     __shared__ unsigned goff[R];
     __shared__ unsigned wcnt[NW][R];
+    __shared__ unsigned wsum[NW];
+    __shared__ unsigned skey[kSortChunk];
+    __shared__ V sval[kSortChunk];
     const unsigned long long n = *d_n;
     const unsigned long long nchunk = (n + kSortChunk - 1) / kSortChunk;
     const int wave = threadIdx.x >> 6;
@@ -661,27 +719,31 @@ void k_sort_scatter(const unsigned* __restrict__ keys_in,
     const unsigned long long lt = lanemask_lt();
     for (unsigned long long c = blockIdx.x; c < nchunk; c += gridDim.x)
     {
-        for (int d = threadIdx.x; d < R; d += kSortThreads)
+        for (int d = threadIdx.x; d < R; d += kScatterThreads)
         {
             goff[d] = hist_off[d * nchunk + c];
             #pragma unroll
             for (int w = 0; w < NW; ++w) wcnt[w][d] = 0;
         }
         __syncthreads();
-        const unsigned long long base = c * kSortChunk + (unsigned long long)wave * (SUB * 64);
-        unsigned key[SUB], val[SUB], rank[SUB];
+        const unsigned long long left = n - c * kSortChunk;
+        const int m = (int)(left < kSortChunk ? left : kSortChunk);
+        const int at0 = wave * (SUB * 64) + lane;         // (in the chunk)
+        const unsigned* kin = keys_in + c * kSortChunk;
+        const V* vin = vals_in + c * kSortChunk;
+        unsigned key[SUB], rank[SUB];
+        V val[SUB];
         #pragma unroll
         for (int r = 0; r < SUB; ++r)
         {
-            const unsigned long long idx = base + r * 64 + lane;
-            const bool valid = idx < n;
-            key[r] = valid ? keys_in[idx] : 0u;
-            val[r] = valid ? vals_in[idx] : 0u;
+            const int idx = at0 + r * 64;
+            key[r] = idx < m ? kin[idx] : 0u;
+            val[r] = idx < m ? vin[idx] : (V)0;
         }
         #pragma unroll
         for (int r = 0; r < SUB; ++r)
         {
-            const bool valid = base + r * 64 + lane < n;
+            const bool valid = at0 + r * 64 < m;
             const unsigned d = (key[r] >> shift) & M;
             unsigned long long peers = __ballot(valid);
             #pragma unroll
@@ -697,27 +759,61 @@ void k_sort_scatter(const unsigned* __restrict__ keys_in,
             if (valid && before == 0) wcnt[wave][d] = prior + (unsigned)__popcll(peers);
         }
         __syncthreads();
-        for (int d = threadIdx.x; d < R; d += kSortThreads)
+        // The chunk's digits in order: each thread kPer of them.
+        constexpr int kPer = (R + kScatterThreads - 1) / kScatterThreads;
+        unsigned mine = 0;
+        #pragma unroll
+        for (int j = 0; j < kPer; ++j)
         {
-            unsigned acc = goff[d];
+            const int d = threadIdx.x * kPer + j;
+            if (d >= R) break;
+            #pragma unroll
+            for (int w = 0; w < NW; ++w) mine += wcnt[w][d];
+        }
+        unsigned run = mine;
+        #pragma unroll
+        for (int o = 1; o < 64; o <<= 1)
+        {
+            const unsigned y = __shfl_up(run, o, 64);
+            if (lane >= o) run += y;
+        }
+        if (lane == 63) wsum[wave] = run;
+        __syncthreads();
+        run -= mine;
+        for (int w = 0; w < wave; ++w) run += wsum[w];
+        #pragma unroll
+        for (int j = 0; j < kPer; ++j)
+        {
+            const int d = threadIdx.x * kPer + j;
+            if (d >= R) break;
+            goff[d] -= run;                       // (position in the output - in the chunk)
             #pragma unroll
             for (int w = 0; w < NW; ++w)
             {
                 const unsigned t = wcnt[w][d];
-                wcnt[w][d] = acc;
-                acc += t;
+                wcnt[w][d] = run;
+                run += t;
             }
         }
         __syncthreads();
         #pragma unroll
         for (int r = 0; r < SUB; ++r)
         {
-            if (base + r * 64 + lane < n)
+            if (at0 + r * 64 < m)
             {
-                const unsigned dst = wcnt[wave][(key[r] >> shift) & M] + rank[r];
-                keys_out[dst] = key[r];
-                vals_out[dst] = val[r];
+                const unsigned at = wcnt[wave][(key[r] >> shift) & M] + rank[r];
+                skey[at] = key[r];
+                sval[at] = val[r];
             }
+        }
+        __syncthreads();
+        #pragma unroll 4
+        for (int i = threadIdx.x; i < m; i += kScatterThreads)
+        {
+            const unsigned k = skey[i];
+            const unsigned dst = goff[(k >> shift) & M] + (unsigned)i;
+            keys_out[dst] = k;
+            vals_out[dst] = sval[i];
         }
         __syncthreads();
     }

@@ -3,8 +3,9 @@
 // the input weights divided by their cell's sum ("read").
 //
 // Write is an ordered floating-point sum per cell, so it runs as
-//   k_weight_cells  key = cell index (or `outside`), value = point index
-//   radix sort      stable, so each cell's points stay in input order
+//   k_weight_cells  key = cell index (or `outside`)
+//   radix sort      of (key, weight), stable: each cell's weights end up side
+//                   by side in input order
 //   k_weight_sum    one thread per cell adds the cell's weights, in input
 //                   order, to the cell's existing value
 // which performs, per cell, exactly the additions of the serial loop in the
@@ -92,7 +93,8 @@ __device__ __forceinline__ void weight_block_flush(unsigned cnt, int u0, int v0,
 }
 
 // Per point: when keys is given, key = v * G + u for points inside the grid
-// and `outside` (> every cell index) for the others, value = point index.
+// and `outside` (> every cell index) for the others, and when vals is given
+// too, value = point index.
 // Counts the points off the grid and, when box is given, the bounding box of
 // the cells in use.  Block size 256.
 template <typename T>
@@ -112,7 +114,7 @@ void k_weight_cells(const T* __restrict__ uu, const T* __restrict__ vv, unsigned
         if (keys)
         {
             keys[i] = in ? (unsigned)gv * (unsigned)grid_size + (unsigned)gu : outside;
-            vals[i] = (unsigned)i;
+            if (vals) vals[i] = (unsigned)i;
         }
         if (in)
         {
@@ -125,30 +127,115 @@ void k_weight_cells(const T* __restrict__ uu, const T* __restrict__ vv, unsigned
     weight_block_flush(cnt, u0, v0, u1, v1, skipped, box);
 }
 
-// Over the stably sorted (key, point) pairs: the first position of each cell
-// adds that cell's weights, in point order, to the cell's value.  The cell
-// (u, v) lives at grid[(v - v0) * pitch + (u - u0)] (a window of the grid
-// starting at cell (u0, v0), or the whole grid with u0 = v0 = 0, pitch = G).
-template <typename T>
-__global__ __launch_bounds__(256)
+// Over the stably sorted keys: adds each cell's weights, in point order, to
+// the cell's value.  The weights lie in the sorted order (BY_INDEX: at
+// vals[]).  The cell (u, v) lives at grid[(v - v0) * pitch + (u - u0)] (a
+// window of the grid starting at cell (u0, v0), or the whole grid with u0 = v0
+// = 0, pitch = G).
+//
+// A cell's additions are a serial chain by contract, and a lane that walks its
+// cell through global memory pays a scattered load per point.  So one wave
+// takes kSumChunk positions: it copies the weights to LDS with coalesced
+// loads, lists the positions where a cell starts (most are not) and then gives
+// each listed cell a lane, which adds from LDS.  The chunk's last cell can run
+// on past it; the wave follows it 64 points at a time, the sum uniform, each
+// weight taken from its lane's register.  31.4M points on 16384^2, longest
+// cell 374 points: 1296 -> 155 us.
+constexpr int kSumChunk = 512;
+
+template <typename T, bool BY_INDEX>
+__global__ __launch_bounds__(64)
 void k_weight_sum(const unsigned* __restrict__ keys, const unsigned* __restrict__ vals,
         const T* __restrict__ weight, unsigned long long n, unsigned outside, int grid_size,
         T* __restrict__ grid, int u0, int v0, unsigned long long pitch)
 {
-    for (unsigned long long p = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
-            p < n; p += (unsigned long long)gridDim.x * blockDim.x)
+    constexpr int kRows = kSumChunk / 64, kAhead = 4;
+    __shared__ T sw[kSumChunk + kAhead];
+    __shared__ unsigned cell[kSumChunk];
+    __shared__ unsigned short start[kSumChunk + 1];
+    __shared__ T tail;
+    const int lane = threadIdx.x;
+    const unsigned long long nchunk = (n + kSumChunk - 1) / kSumChunk;
+    for (unsigned long long c = blockIdx.x; c < nchunk; c += gridDim.x)
     {
-        const unsigned k = keys[p];
-        if (k == outside || (p > 0 && keys[p - 1] == k)) continue;
-        unsigned long long e = p + 1;
-        while (e < n && keys[e] == k) ++e;
-        const unsigned cv = k / (unsigned)grid_size;
-        const unsigned cu = k - cv * (unsigned)grid_size;
-        T* cell = grid + (unsigned long long)(cv - (unsigned)v0) * pitch + (cu - (unsigned)u0);
-        T acc = *cell;
-        #pragma unroll 4
-        for (unsigned long long q = p; q < e; ++q) acc += weight[vals[q]];
-        *cell = acc;
+        const unsigned long long base = c * kSumChunk;
+        const int m = (int)(n - base < kSumChunk ? n - base : kSumChunk);
+        unsigned key[kRows];
+        T w[kRows];
+        #pragma unroll
+        for (int r = 0; r < kRows; ++r)
+        {
+            const unsigned long long i = base + r * 64 + lane;
+            key[r] = i < n ? keys[i] : outside;
+            w[r] = i < n ? weight[BY_INDEX ? vals[i] : i] : (T)0;
+        }
+        // (`outside` is the largest key: those points come last and start no cell.)
+        unsigned last = base > 0 ? keys[base - 1] : outside;
+        int cells = 0, end = 0;
+        #pragma unroll
+        for (int r = 0; r < kRows; ++r)
+        {
+            unsigned before = (unsigned)__shfl_up((int)key[r], 1, 64);
+            if (lane == 0) before = last;
+            last = (unsigned)__builtin_amdgcn_readlane((int)key[r], 63);
+            const bool in = key[r] != outside;
+            const bool first = in && key[r] != before;
+            const unsigned long long f = __ballot(first);
+            if (first)
+            {
+                const int at = cells + __popcll(f & lanemask_lt());
+                start[at] = (unsigned short)(r * 64 + lane);
+                cell[at] = key[r];
+            }
+            cells += __popcll(f);
+            end += __popcll(__ballot(in));
+            sw[r * 64 + lane] = w[r];
+        }
+        if (lane == 0) start[cells] = (unsigned short)end;
+        __syncthreads();
+        for (int j = lane; j < cells; j += 64)
+        {
+            const unsigned k = cell[j];
+            const unsigned cv = k / (unsigned)grid_size, cu = k - cv * (unsigned)grid_size;
+            T* at = grid + (unsigned long long)(cv - (unsigned)v0) * pitch + (cu - (unsigned)u0);
+            T acc = *at;
+            const int e = start[j + 1];
+            for (int q = start[j]; q < e; q += kAhead)
+            {
+                T x[kAhead];
+                #pragma unroll
+                for (int i = 0; i < kAhead; ++i) x[i] = sw[q + i];
+                #pragma unroll
+                for (int i = 0; i < kAhead; ++i) if (q + i < e) acc += x[i];
+            }
+            *at = acc;
+            if (j == cells - 1) tail = acc;
+        }
+        __syncthreads();
+        // Past the chunk: only where the chunk is full and its last cell goes on.
+        if (cells && end == kSumChunk && base + kSumChunk < n)
+        {
+            const unsigned k = last;
+            const unsigned long long q0 = base + kSumChunk;
+            if (keys[q0] == k)
+            {
+                const unsigned cv = k / (unsigned)grid_size, cu = k - cv * (unsigned)grid_size;
+                T* at = grid + (unsigned long long)(cv - (unsigned)v0) * pitch
+                        + (cu - (unsigned)u0);
+                T acc = tail;
+                int more = 64;
+                for (unsigned long long q = q0; more == 64; q += 64)
+                {
+                    const unsigned long long i = q + lane;
+                    const bool in = i < n && keys[i] == k;
+                    const T x = in ? weight[BY_INDEX ? vals[i] : i] : (T)0;
+                    more = __popcll(__ballot(in));
+                    for (int l = 0; l < more; ++l) acc += read_lane(x, l);
+                }
+                if (lane == 0) *at = acc;
+            }
+        }
+        __syncthreads();
     }
 }
 

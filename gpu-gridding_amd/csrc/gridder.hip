@@ -713,14 +713,35 @@ enum Scalar { SC_VISITS, SC_OVERFLOW, SC_ITEMS, SC_SLOTS, SC_SCRATCH0, SC_RUNS =
 
 // Stable LSD radix sort of the pairs (C->keys[0], C->vals[0]) on the low
 // key_bits bits of the keys: *d_n pairs, n_bound an upper bound of *d_n
-// known on the host.  Digits are 8 bits, or 9 where that saves a pass (27
-// bits in 3 passes instead of 4).  *cur receives the index of the
-// ping-pong buffers holding the result.
+// known on the host.  The values are Vs, read in the first pass from `first`
+// where that is given.  Digits are 8 bits, or 9 where that saves a pass (27
+// bits in 3 passes instead of 4; 10 bits would save one at 29 and 30 bits, but
+// their passes take 385 us each where the four of 8 bits take 206: 31.4M
+// pairs).  *cur receives the index of the ping-pong buffers holding the
+// result.
+template <int BITS, typename V>
+int radix_pass(mi355_ctx* C, unsigned long long nchunk, const unsigned long long* d_n, int shift,
+        int cur, const V* vals)
+{
+    unsigned long long* sc = C->scalars.as<unsigned long long>();
+    const unsigned radix = 1u << BITS, blocks = grid_blocks(nchunk, 1, 16384);
+    hipLaunchKernelGGL(k_sort_hist<BITS>, dim3(blocks), dim3(kSortThreads), 0, C->stream,
+            C->keys[cur].as<unsigned>(), d_n, shift, C->hist.as<unsigned>());
+    DevCount hc{d_n, (unsigned long long)kSortChunk, radix, 0};
+    TRY(scan_u32(C, C->hist.as<unsigned>(), C->hist_off.as<unsigned>(), hc, radix * nchunk,
+            sc + SC_SCRATCH0, reinterpret_cast<unsigned*>(sc + SC_SCRATCH0 + 1), 0));
+    hipLaunchKernelGGL((k_sort_scatter<BITS, V>), dim3(blocks), dim3(kScatterThreads), 0, C->stream,
+            C->keys[cur].as<unsigned>(), vals, d_n, shift, C->hist_off.as<unsigned>(),
+            C->keys[cur ^ 1].as<unsigned>(), C->vals[cur ^ 1].as<V>());
+    HIP_TRY(hipGetLastError());
+    return MI355_OK;
+}
+
+template <typename V>
 int radix_sort(mi355_ctx* C, unsigned long long n_bound, const unsigned long long* d_n,
-        int key_bits, int* cur_out)
+        int key_bits, const V* first, int* cur_out)
 {
     C->bk_valid = false;              // (the ping-pong buffers are rewritten)
-    unsigned long long* sc = C->scalars.as<unsigned long long>();
     const int bits = (key_bits + 8) / 9 < (key_bits + 7) / 8 ? 9 : 8;
     const unsigned radix = 1u << bits;
     const unsigned long long nchunk = (n_bound + kSortChunk - 1) / kSortChunk;
@@ -729,27 +750,9 @@ int radix_sort(mi355_ctx* C, unsigned long long n_bound, const unsigned long lon
     int cur = 0;
     for (int shift = 0; shift < key_bits; shift += bits)
     {
-        const unsigned blocks = grid_blocks(nchunk, 1, 16384);
-        if (bits == 9)
-            hipLaunchKernelGGL(k_sort_hist<9>, dim3(blocks), dim3(kSortThreads), 0, C->stream,
-                    C->keys[cur].as<unsigned>(), d_n, shift, C->hist.as<unsigned>());
-        else
-            hipLaunchKernelGGL(k_sort_hist<8>, dim3(blocks), dim3(kSortThreads), 0, C->stream,
-                    C->keys[cur].as<unsigned>(), d_n, shift, C->hist.as<unsigned>());
-        DevCount hc{d_n, (unsigned long long)kSortChunk, radix, 0};
-        TRY(scan_u32(C, C->hist.as<unsigned>(), C->hist_off.as<unsigned>(), hc, radix * nchunk,
-                sc + SC_SCRATCH0, reinterpret_cast<unsigned*>(sc + SC_SCRATCH0 + 1), 0));
-        if (bits == 9)
-            hipLaunchKernelGGL(k_sort_scatter<9>, dim3(blocks), dim3(kSortThreads), 0, C->stream,
-                    C->keys[cur].as<unsigned>(), C->vals[cur].as<unsigned>(), d_n, shift,
-                    C->hist_off.as<unsigned>(), C->keys[cur ^ 1].as<unsigned>(),
-                    C->vals[cur ^ 1].as<unsigned>());
-        else
-            hipLaunchKernelGGL(k_sort_scatter<8>, dim3(blocks), dim3(kSortThreads), 0, C->stream,
-                    C->keys[cur].as<unsigned>(), C->vals[cur].as<unsigned>(), d_n, shift,
-                    C->hist_off.as<unsigned>(), C->keys[cur ^ 1].as<unsigned>(),
-                    C->vals[cur ^ 1].as<unsigned>());
-        HIP_TRY(hipGetLastError());
+        const V* vals = shift == 0 && first ? first : C->vals[cur].as<V>();
+        TRY(bits == 9 ? (radix_pass<9, V>(C, nchunk, d_n, shift, cur, vals))
+                      : (radix_pass<8, V>(C, nchunk, d_n, shift, cur, vals)));
         cur ^= 1;
     }
     *cur_out = cur;
@@ -1061,7 +1064,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     HIP_TRY(hipGetLastError());
     const int key_bits = tile_bits + key_table_bits;
     int cur = 0;
-    TRY(radix_sort(C, T_vis, sc + SC_VISITS, key_bits, &cur));
+    TRY(radix_sort<unsigned>(C, T_vis, sc + SC_VISITS, key_bits, nullptr, &cur));
     const unsigned* skeys = C->keys[cur].as<unsigned>();
     // (for mi355_ctx_get_buckets: where this pass's sorted lists are)
     C->bk_valid = f32 && (strips || bands) && !C->sync_free;
@@ -1687,7 +1690,7 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
                 C->keys[0].as<unsigned>(), C->vals[0].as<unsigned>());
         HIP_TRY(hipGetLastError());
         int cur = 0;
-        TRY(radix_sort(C, N, sc + SC_VISITS, bits_for(ntile + 1), &cur));
+        TRY(radix_sort<unsigned>(C, N, sc + SC_VISITS, bits_for(ntile + 1), nullptr, &cur));
         order = C->vals[cur].as<unsigned>();
     }
     hipLaunchKernelGGL(k_degrid<T>, dim3(grid_blocks(N, 4, 65535)), dim3(256), 0, C->stream,
@@ -1760,25 +1763,54 @@ int check_weights_args(size_t N, int G)
     return MI355_OK;
 }
 
-// Cell keys of the N points, stably sorted (point order kept within a cell);
-// counts points off the grid into *skipped and the cells' bounding box into
-// box (when given).  Expects k_weight_init to have set SC_W_COUNT to N.
+// Cell keys of the N points and their weights, stably sorted (point order
+// kept within a cell); counts points off the grid into *skipped and the
+// cells' bounding box into box (when given).  Expects k_weight_init to have
+// set SC_W_COUNT to N.  The weights themselves go through the sort, so that
+// each cell's lie side by side for its sum; FP64 ones need 8 bytes more per
+// point than indices would, and under a workspace cap indices go instead.
 template <typename T>
-int weights_sorted_cells(mi355_ctx* C, size_t N, const T* uu, const T* vv, T gs, int G,
-        unsigned long long* skipped, int* box, int* cur)
+bool weights_by_index(const mi355_ctx* C) { return sizeof(T) == 8 && C->max_workspace; }
+
+template <typename T>
+int weights_sorted_cells(mi355_ctx* C, size_t N, const T* uu, const T* vv, const T* weight, T gs,
+        int G, unsigned long long* skipped, int* box, int* cur)
 {
+    typedef typename std::conditional<sizeof(T) == 8, unsigned long long, unsigned>::type Bits;
+    const bool by_index = weights_by_index<T>(C);
     for (int b = 0; b < 2; ++b)
     {
         TRY(ensure(C, C->keys[b], N * sizeof(unsigned)));
-        TRY(ensure(C, C->vals[b], N * sizeof(unsigned)));
+        TRY(ensure(C, C->vals[b], N * (by_index ? sizeof(unsigned) : sizeof(T))));
     }
     const unsigned long long cells = (unsigned long long)G * G;
     hipLaunchKernelGGL(k_weight_cells<T>, dim3(grid_blocks(N, 256, 16384)), dim3(256), 0,
             C->stream, uu, vv, (unsigned long long)N, gs, G, (unsigned)cells,
-            C->keys[0].as<unsigned>(), C->vals[0].as<unsigned>(), skipped, box);
+            C->keys[0].as<unsigned>(), by_index ? C->vals[0].as<unsigned>() : nullptr, skipped, box);
     HIP_TRY(hipGetLastError());
-    return radix_sort(C, N, C->scalars.as<unsigned long long>() + SC_W_COUNT,
-            bits_for(cells + 1), cur);
+    const unsigned long long* d_n = C->scalars.as<unsigned long long>() + SC_W_COUNT;
+    const int bits = bits_for(cells + 1);
+    return by_index ? radix_sort<unsigned>(C, N, d_n, bits, nullptr, cur)
+                    : radix_sort<Bits>(C, N, d_n, bits, reinterpret_cast<const Bits*>(weight), cur);
+}
+
+// The sums over the sorted pairs, into the window of the grid given.
+template <typename T>
+int weights_sums(mi355_ctx* C, size_t N, const T* weight, int G, int cur, T* grid, int u0, int v0,
+        unsigned long long pitch)
+{
+    const dim3 blocks(grid_blocks(N, kSumChunk, 1 << 20));
+    const unsigned outside = (unsigned)((unsigned long long)G * G);
+    if (weights_by_index<T>(C))
+        hipLaunchKernelGGL((k_weight_sum<T, true>), blocks, dim3(64), 0, C->stream,
+                C->keys[cur].as<unsigned>(), C->vals[cur].as<unsigned>(), weight,
+                (unsigned long long)N, outside, G, grid, u0, v0, pitch);
+    else
+        hipLaunchKernelGGL((k_weight_sum<T, false>), blocks, dim3(64), 0, C->stream,
+                C->keys[cur].as<unsigned>(), (const unsigned*)nullptr, C->vals[cur].as<T>(),
+                (unsigned long long)N, outside, G, grid, u0, v0, pitch);
+    HIP_TRY(hipGetLastError());
+    return MI355_OK;
 }
 
 template <typename T>
@@ -1797,12 +1829,8 @@ int weights_write_dev(mi355_ctx* C, size_t N, const T* uu, const T* vv, const T*
     if (N == 0) return ok();
     const T gs = (T)G * cell;     // oskar_grid_weights.c:113 / :44
     int cur = 0;
-    TRY(weights_sorted_cells<T>(C, N, uu, vv, gs, G, skipped, nullptr, &cur));
-    hipLaunchKernelGGL(k_weight_sum<T>, dim3(grid_blocks(N, 256, 65535)), dim3(256), 0,
-            C->stream, C->keys[cur].as<unsigned>(), C->vals[cur].as<unsigned>(), weight,
-            (unsigned long long)N, (unsigned)((unsigned long long)G * G), G, grid, 0, 0,
-            (unsigned long long)G);
-    HIP_TRY(hipGetLastError());
+    TRY(weights_sorted_cells<T>(C, N, uu, vv, weight, gs, G, skipped, nullptr, &cur));
+    TRY(weights_sums<T>(C, N, weight, G, cur, grid, 0, 0, (unsigned long long)G));
     return ok();
 }
 
@@ -1866,8 +1894,8 @@ int weights_write_host(size_t N, const T* uu, const T* vv, const T* weight, T ce
             (unsigned long long)N, skipped, box);
     const T gs = (T)G * cell;
     int cur = 0;
-    TRY(weights_sorted_cells<T>(C, N, C->in_uu.as<T>(), C->in_vv.as<T>(), gs, G, skipped, box,
-            &cur));
+    TRY(weights_sorted_cells<T>(C, N, C->in_uu.as<T>(), C->in_vv.as<T>(), C->in_weight.as<T>(), gs,
+            G, skipped, box, &cur));
     int hbox[4];
     unsigned long long hskip = 0;
     HIP_TRY(hipMemcpyAsync(hbox, box, sizeof(hbox), hipMemcpyDeviceToHost, C->stream));
@@ -1877,12 +1905,8 @@ int weights_write_host(size_t N, const T* uu, const T* vv, const T* weight, T ce
     {
         TRY(upload_weight_window<T>(C, grid, G, hbox));
         const size_t ww = (size_t)(hbox[2] - hbox[0] + 1), wh = (size_t)(hbox[3] - hbox[1] + 1);
-        hipLaunchKernelGGL(k_weight_sum<T>, dim3(grid_blocks(N, 256, 65535)), dim3(256), 0,
-                C->stream, C->keys[cur].as<unsigned>(), C->vals[cur].as<unsigned>(),
-                C->in_weight.as<T>(), (unsigned long long)N,
-                (unsigned)((unsigned long long)G * G), G, C->in_grid.as<T>(), hbox[0], hbox[1],
-                (unsigned long long)ww);
-        HIP_TRY(hipGetLastError());
+        TRY(weights_sums<T>(C, N, C->in_weight.as<T>(), G, cur, C->in_grid.as<T>(), hbox[0],
+                hbox[1], (unsigned long long)ww));
         TRY(stage_download(C, grid + (size_t)hbox[1] * G + hbox[0], (size_t)G * sizeof(T),
                 C->in_grid.p, ww * sizeof(T), ww * sizeof(T), wh));
     }
