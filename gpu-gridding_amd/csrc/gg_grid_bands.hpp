@@ -51,7 +51,7 @@ struct BandCfg
     static constexpr int kUnitBytes = 8 * kLaneBytes;
     static constexpr int kStride = kBlockW / kLaneCells + 8; // 16-byte words per LDS row
     static constexpr int kMaxUnits = kBlockW / kUnitW + 1;  // units of one row in a block
-    static_assert(kRegionW * kRegionH % kMergeCells == 0, "merge blocks tile a region");
+    static_assert(kRegionW * kRegionH % kMergeCells<float2> == 0, "merge blocks tile a region");
     static_assert(kWork == 32, "shares of an item, whatever the precision");
 };
 

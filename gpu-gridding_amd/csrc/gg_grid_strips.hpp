@@ -78,7 +78,7 @@ struct StripCfg
     static constexpr int kDirectGroup = COMP ? GG_DIRECT_GROUP_COMP : GG_DIRECT_GROUP;
     static constexpr bool kComp = COMP;
     static_assert(ROWS % 16 == 0 && ROWS <= 128, "blocks of 16 rows, two LDS bases of 64 rows");
-    static_assert(kRegionW * kRegionH % kMergeCells == 0, "merge blocks tile a region");
+    static_assert(kRegionW * kRegionH % kMergeCells<float2> == 0, "merge blocks tile a region");
 };
 using StripPlain = StripCfg<GG_STRIP_WAVES, 128, false>;
 using StripComp = StripCfg<12, 64, true>;
