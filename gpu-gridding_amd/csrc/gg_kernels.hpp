@@ -481,6 +481,29 @@ __device__ __forceinline__ void scan_load(const unsigned* __restrict__ in,
     for (int q = 0; q < kScanPerThread; ++q) vals[q] = base + q < n ? in[base + q] : 0u;
 }
 
+// ... and their exclusive sums from `run` on, stored likewise.
+__device__ __forceinline__ void scan_store(unsigned* __restrict__ out, unsigned long long base,
+        unsigned long long n, unsigned (&vals)[kScanPerThread], unsigned long long run)
+{
+    #pragma unroll
+    for (int q = 0; q < kScanPerThread; ++q)
+    {
+        const unsigned x = vals[q];
+        vals[q] = (unsigned)run;
+        run += x;
+    }
+    if (base + kScanPerThread <= n)
+    {
+        #pragma unroll
+        for (int q = 0; q < kScanPerThread; q += 4)
+            *reinterpret_cast<uint4*>(out + base + q) =
+                    make_uint4(vals[q], vals[q + 1], vals[q + 2], vals[q + 3]);
+        return;
+    }
+    #pragma unroll
+    for (int q = 0; q < kScanPerThread; ++q) if (base + q < n) out[base + q] = vals[q];
+}
+
 __global__ __launch_bounds__(kScanThreads)
 void k_scan_reduce(const unsigned* __restrict__ in, DevCount cnt,
         unsigned long long* __restrict__ partial)
@@ -560,26 +583,59 @@ void k_scan_down(const unsigned* __restrict__ in, DevCount cnt,
         #pragma unroll
         for (int q = 0; q < kScanPerThread; ++q) s += vals[q];
         unsigned long long tot;
-        unsigned long long run = partial[c] + block_excl_scan_u64(s, sh, &tot);
+        scan_store(out, base, n, vals, partial[c] + block_excl_scan_u64(s, sh, &tot));
+    }
+}
+
+// The whole scan by one workgroup, 16384 elements a round: workgroup 0 scans
+// in0, workgroup 1 (where launched) in1.  For arrays short enough that the
+// three kernels above are all launch and no work.
+constexpr unsigned long long kScanSmallMax = 32768;
+
+__global__ __launch_bounds__(1024)
+void k_scan_small(DevCount cnt, const unsigned* __restrict__ in0, unsigned* __restrict__ out0,
+        unsigned long long* __restrict__ total0, const unsigned* __restrict__ in1,
+        unsigned* __restrict__ out1, unsigned long long* __restrict__ total1,
+        unsigned* __restrict__ overflow, int write_end)
+{
+    __shared__ unsigned long long sh[16];
+    const unsigned* in = blockIdx.x ? in1 : in0;
+    unsigned* out = blockIdx.x ? out1 : out0;
+    const unsigned long long n = cnt.get();
+    const int lane = lane_id(), wave = threadIdx.x >> 6;
+    unsigned long long done = 0;                   // sum of the rounds before
+    for (unsigned long long c = 0; c < n; c += 1024 * kScanPerThread)
+    {
+        const unsigned long long base = c + (unsigned long long)threadIdx.x * kScanPerThread;
+        unsigned vals[kScanPerThread];
+        scan_load(in, base, n, vals);
+        unsigned long long s = 0;
         #pragma unroll
-        for (int q = 0; q < kScanPerThread; ++q)
+        for (int q = 0; q < kScanPerThread; ++q) s += vals[q];
+        unsigned long long v = s;
+        #pragma unroll
+        for (int o = 1; o < 64; o <<= 1)
         {
-            const unsigned x = vals[q];
-            vals[q] = (unsigned)run;
-            run += x;
+            const unsigned long long y = __shfl_up(v, o, 64);
+            if (lane >= o) v += y;
         }
-        if (base + kScanPerThread <= n)
+        if (lane == 63) sh[wave] = v;
+        __syncthreads();
+        unsigned long long run = done + v - s;
+        #pragma unroll
+        for (int w = 0; w < 16; ++w)
         {
-            #pragma unroll
-            for (int q = 0; q < kScanPerThread; q += 4)
-                *reinterpret_cast<uint4*>(out + base + q) =
-                        make_uint4(vals[q], vals[q + 1], vals[q + 2], vals[q + 3]);
+            if (w < wave) run += sh[w];
+            done += sh[w];
         }
-        else
-        {
-            #pragma unroll
-            for (int q = 0; q < kScanPerThread; ++q) if (base + q < n) out[base + q] = vals[q];
-        }
+        __syncthreads();
+        scan_store(out, base, n, vals, run);
+    }
+    if (threadIdx.x == 0)
+    {
+        *(blockIdx.x ? total1 : total0) = done;
+        if (done > 0xFFFFFFFFull) *overflow = 1u;
+        if (write_end) out[n] = (unsigned)done;
     }
 }
 
@@ -827,6 +883,15 @@ __global__ void k_fill_u32(unsigned* __restrict__ p, unsigned long long n, unsig
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
             i < n; i += (unsigned long long)gridDim.x * blockDim.x)
         p[i] = v;
+}
+
+// Two ranges in one launch: a's words to va, b's to vb.
+__global__ void k_fill2_u32(unsigned* __restrict__ a, unsigned long long na,
+        unsigned* __restrict__ b, unsigned long long nb, unsigned va, unsigned vb)
+{
+    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
+            i < na + nb; i += (unsigned long long)gridDim.x * blockDim.x)
+        if (i < na) a[i] = va; else b[i - na] = vb;
 }
 
 __global__ void k_tile_bounds(const unsigned* __restrict__ keys,

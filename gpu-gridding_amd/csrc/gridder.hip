@@ -234,18 +234,18 @@ struct mi355_ctx
     unsigned long long table_tail = 0;
     int max_support = 0;
 
-    DevBuf tables, norm_table, support_d, plane_off_d;
+    DevBuf tables, norm_table, support_d;   // (support_d: supports, then table offsets)
     DevBuf meta, amp, num_visits, visit_off;
     DevBuf part_norm, part_skipped, part_taps, part_nonfinite, part_bbox;
     DevBuf scan_partial, scalars;
     DevBuf keys[2], vals[2], hist, hist_off;
-    DevBuf tile_start, tile_end, n_items, n_slots, item_off, slot_off, item_tile;
+    DevBuf tile_bounds, n_items, n_slots, item_off, slot_off, item_tile;
     DevBuf run_start, run_z, run_tb;
     DevBuf vmeta, vamp, vlds;       // sorted visit records (strip and band kernels)
     DevBuf vrec;                    // per-visibility record + amplitude (their gathers)
     DevBuf band_items, order_count; // band kernel: its items, and their counts by first table
     DevBuf scratch;
-    DevBuf jobs_d, job_chunk_off_d, job_vis_off_d, job_tile_base_d, job_out_d, job_bbox_d, job_norm_d;
+    DevBuf jobs_d, job_norm_d;         // (jobs_d: see JobLayout)
     // drop-in staging
     DevBuf in_conv, in_uu, in_vv, in_ww, in_vis, in_weight, in_grid, in_norm, in_skipped;
     DevBuf in_weight_out;
@@ -261,10 +261,8 @@ struct mi355_ctx
 
     // host mirrors kept alive across asynchronous uploads
     std::vector<unsigned char> h_jobs;
-    std::vector<unsigned> h_job_chunk_off, h_job_tile_base;
-    std::vector<unsigned long long> h_job_vis_off;
-    std::vector<unsigned long long> h_job_out;
-    std::vector<int4> h_job_bbox;
+    std::vector<int> h_planes;
+    std::vector<unsigned long long> h_scalars;   // (a download's)
 
     hipEvent_t ev[EV_COUNT] = {};
     mi355_stats stats = {};
@@ -534,15 +532,14 @@ int init_ctx(mi355_ctx* C, int device)
 // Every device buffer a context holds.
 std::vector<DevBuf*> device_buffers(mi355_ctx* C)
 {
-    return {&C->tables, &C->norm_table, &C->support_d, &C->plane_off_d, &C->meta,
+    return {&C->tables, &C->norm_table, &C->support_d, &C->meta,
         &C->amp, &C->num_visits, &C->visit_off, &C->part_norm, &C->part_skipped,
         &C->part_taps, &C->part_nonfinite, &C->part_bbox, &C->scan_partial, &C->scalars,
         &C->keys[0], &C->keys[1],
-        &C->vals[0], &C->vals[1], &C->hist, &C->hist_off, &C->tile_start, &C->tile_end,
+        &C->vals[0], &C->vals[1], &C->hist, &C->hist_off, &C->tile_bounds,
         &C->n_items, &C->n_slots, &C->item_off, &C->slot_off, &C->item_tile, &C->run_start,
         &C->run_z, &C->run_tb, &C->scratch,
-        &C->jobs_d, &C->job_chunk_off_d, &C->job_vis_off_d, &C->job_tile_base_d,
-        &C->job_out_d, &C->job_bbox_d, &C->job_norm_d, &C->in_conv, &C->in_uu, &C->in_vv, &C->in_ww,
+        &C->jobs_d, &C->job_norm_d, &C->in_conv, &C->in_uu, &C->in_vv, &C->in_ww,
         &C->in_vis, &C->in_weight, &C->in_grid, &C->in_norm, &C->in_skipped, &C->in_weight_out,
         &C->fft_work, &C->in_image, &C->vmeta, &C->vamp, &C->vlds, &C->vrec,
         &C->band_items, &C->order_count};
@@ -605,6 +602,8 @@ int check_grid_args(int grid_size)
 // ---------------------------------------------------------------------------
 // Kernel tables
 // ---------------------------------------------------------------------------
+const unsigned* plane_offsets(const mi355_ctx* C, size_t P) { return C->support_d.as<unsigned>() + P; }
+
 template <typename TI, typename TA>
 int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         const typename V2<TI>::t* conv_dev, int lane_cells)
@@ -644,23 +643,21 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     TRY(ensure(C, C->tables, (off + tail) * sizeof(T2)));
     C->table_tail = tail;
     {
-        // zero the guard and the tail (fill kernels: no memset nodes)
+        // zero the guard and the tail (a fill kernel: no memset nodes)
         const unsigned wpe = sizeof(T2) / 4;
-        hipLaunchKernelGGL(k_fill_u32, dim3(grid_blocks(guard * wpe, 256, 1024)), dim3(256), 0,
-                C->stream, C->tables.as<unsigned>(), guard * wpe, 0u);
-        hipLaunchKernelGGL(k_fill_u32, dim3(grid_blocks(tail * wpe, 256, 1024)), dim3(256), 0,
-                C->stream, reinterpret_cast<unsigned*>(C->tables.as<T2>() + off), tail * wpe, 0u);
+        hipLaunchKernelGGL(k_fill2_u32, dim3(grid_blocks((guard + tail) * wpe, 256, 1024)), dim3(256),
+                0, C->stream, C->tables.as<unsigned>(), guard * wpe,
+                reinterpret_cast<unsigned*>(C->tables.as<T2>() + off), tail * wpe, 0u, 0u);
         HIP_TRY(hipGetLastError());
     }
     TRY(ensure(C, C->norm_table, P * (2 * half + 1) * (2 * half + 1) * sizeof(double)));
-    TRY(ensure(C, C->support_d, P * sizeof(int)));
-    TRY(ensure(C, C->plane_off_d, P * sizeof(unsigned)));
+    TRY(ensure(C, C->support_d, 2 * P * sizeof(int)));
     C->cache_support.assign(support, support + P);
+    C->h_planes.assign(support, support + P);
+    for (unsigned o : C->plane_off) C->h_planes.push_back((int)o);
     if (!C->capturing)   // (a captured pipeline reuses what the eager run uploaded)
     {
-        HIP_TRY(hipMemcpyAsync(C->support_d.p, C->cache_support.data(), P * sizeof(int),
-                hipMemcpyHostToDevice, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->plane_off_d.p, C->plane_off.data(), P * sizeof(unsigned),
+        HIP_TRY(hipMemcpyAsync(C->support_d.p, C->h_planes.data(), 2 * P * sizeof(int),
                 hipMemcpyHostToDevice, C->stream));
     }
     {
@@ -669,7 +666,7 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         dim3 g(grid_blocks(rows_max, 4, 16), (unsigned)std::min<size_t>(P, 65535));
         hipLaunchKernelGGL((k_expand_tables<TI, TA>), g, dim3(256), 0, C->stream,
                 conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-                C->plane_off_d.as<unsigned>(), lane_cells, C->tables.as<T2>());
+                plane_offsets(C, P), lane_cells, C->tables.as<T2>());
         HIP_TRY(hipGetLastError());
         const unsigned entries = (unsigned)(P * noff * noff);   // (|off_u|, |off_v|) per plane
         hipLaunchKernelGGL(k_norm_table<TI>, dim3(grid_blocks(entries, 4, 65535)), dim3(256), 0,
@@ -689,20 +686,52 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
 // ---------------------------------------------------------------------------
 // Exclusive scan of n unsigned values (n given on the host or the device)
 // ---------------------------------------------------------------------------
-int scan_u32(mi355_ctx* C, const unsigned* in, unsigned* out, DevCount cnt,
-        unsigned long long n_bound, unsigned long long* d_total, unsigned* d_overflow,
-        int write_end)
+struct ScanJob
 {
+    const unsigned* in;
+    unsigned* out;
+    unsigned long long* d_total;
+};
+
+// Up to two arrays of one length.  Short ones take one kernel, a workgroup
+// each: 3.7 us where the three of the long form take 7.2 and two gaps more (two
+// arrays 4.0 us; a 2k-visibility call 254 -> 208 us, with its uploads and fills
+// joined).  A round of 16384 elements more costs what a launch does, so the
+// line is two rounds.
+int scan_u32(mi355_ctx* C, const ScanJob* jobs, int count, DevCount cnt, unsigned long long n_bound,
+        unsigned* d_overflow, int write_end)
+{
+    if (n_bound <= kScanSmallMax)
+    {
+        const ScanJob& b = jobs[count - 1];
+        hipLaunchKernelGGL(k_scan_small, dim3(count), dim3(1024), 0, C->stream, cnt, jobs[0].in,
+                jobs[0].out, jobs[0].d_total, b.in, b.out, b.d_total, d_overflow, write_end);
+        HIP_TRY(hipGetLastError());
+        return MI355_OK;
+    }
     const unsigned long long nchunk = (n_bound + kScanChunk - 1) / kScanChunk;
     TRY(ensure(C, C->scan_partial, (nchunk + 1) * sizeof(unsigned long long)));
     unsigned long long* part = C->scan_partial.as<unsigned long long>();
     const unsigned blocks = grid_blocks(nchunk, 1, 16384);
-    hipLaunchKernelGGL(k_scan_reduce, dim3(blocks), dim3(kScanThreads), 0, C->stream, in, cnt, part);
-    hipLaunchKernelGGL(k_scan_spine, dim3(1), dim3(1024), 0, C->stream, cnt, part, d_total,
-            d_overflow, out, write_end);
-    hipLaunchKernelGGL(k_scan_down, dim3(blocks), dim3(kScanThreads), 0, C->stream, in, cnt, part, out);
-    HIP_TRY(hipGetLastError());
+    for (const ScanJob* j = jobs; j < jobs + count; ++j)
+    {
+        hipLaunchKernelGGL(k_scan_reduce, dim3(blocks), dim3(kScanThreads), 0, C->stream, j->in,
+                cnt, part);
+        hipLaunchKernelGGL(k_scan_spine, dim3(1), dim3(1024), 0, C->stream, cnt, part, j->d_total,
+                d_overflow, j->out, write_end);
+        hipLaunchKernelGGL(k_scan_down, dim3(blocks), dim3(kScanThreads), 0, C->stream, j->in, cnt,
+                part, j->out);
+        HIP_TRY(hipGetLastError());
+    }
     return MI355_OK;
+}
+
+int scan_u32(mi355_ctx* C, const unsigned* in, unsigned* out, DevCount cnt,
+        unsigned long long n_bound, unsigned long long* d_total, unsigned* d_overflow,
+        int write_end)
+{
+    const ScanJob job{in, out, d_total};
+    return scan_u32(C, &job, 1, cnt, n_bound, d_overflow, write_end);
 }
 
 // Device scalars (u64 slots in C->scalars).  The weighting entry points use
@@ -774,6 +803,31 @@ struct JobHost
     unsigned long long* skipped;
 };
 
+// The job table and the per-job offsets, one buffer and one upload: the jobs,
+// then num_jobs + 1 first visibilities, first selection chunks and first tiles.
+struct JobLayout
+{
+    size_t vis, chunk, tile, bytes;
+    JobLayout(size_t job_bytes, size_t num_jobs)
+        : vis((job_bytes * num_jobs + 7) & ~(size_t)7),
+          chunk(vis + (num_jobs + 1) * sizeof(unsigned long long)),
+          tile(chunk + (num_jobs + 1) * sizeof(unsigned)),
+          bytes(tile + (num_jobs + 1) * sizeof(unsigned)) {}
+    unsigned long long* vis_off(void* p) const { return at<unsigned long long>(p, vis); }
+    unsigned* chunk_off(void* p) const { return at<unsigned>(p, chunk); }
+    unsigned* tile_base(void* p) const { return at<unsigned>(p, tile); }
+    template <typename X> static X* at(void* p, size_t o)
+    {
+        return reinterpret_cast<X*>(static_cast<unsigned char*>(p) + o);
+    }
+};
+
+// The device scalars of a gridding pass and, behind them, what each job counts
+// (skipped, taps, non-finite) and its bounding box: one buffer, one download.
+size_t job_bbox_slot(size_t num_jobs) { return SC_COUNT + ((3 * num_jobs + 1) & ~(size_t)1); }
+size_t scalar_slots(size_t num_jobs) { return job_bbox_slot(num_jobs) + 2 * num_jobs; }
+static_assert(sizeof(int4) == 16 && SC_COUNT % 2 == 0, "a box is two slots, 16-byte aligned");
+
 // Visibilities with non-finite weighted amplitudes (counted by selection),
 // gridded after the tiled path on the same stream.
 template <typename T>
@@ -785,8 +839,8 @@ int grid_nonfinite(mi355_ctx* C, unsigned long long count, int num_jobs,
     typedef typename V4<T>::t T4;
     hipLaunchKernelGGL(k_grid_nonfinite<T>, dim3(grid_blocks(n_total, 4, 65535)), dim3(256), 0,
             C->stream, C->tables.as<T2>(), C->meta.as<int4>(), C->amp.as<T4>(),
-            C->jobs_d.as<JobDev<T>>(), C->job_vis_off_d.as<unsigned long long>(), num_jobs,
-            n_total, C->job_out_d.as<unsigned long long>(), lane_cells);
+            C->jobs_d.as<JobDev<T>>(), JobLayout(sizeof(JobDev<T>), num_jobs).vis_off(C->jobs_d.p),
+            num_jobs, n_total, C->scalars.as<unsigned long long>() + SC_COUNT, lane_cells);
     HIP_TRY(hipGetLastError());
     return MI355_OK;
 }
@@ -798,7 +852,7 @@ int commit_jobs(mi355_ctx* C, int num_jobs)
 {
     hipLaunchKernelGGL(k_job_commit<T>, dim3(grid_blocks(num_jobs, 64, 1024)), dim3(64), 0,
             C->stream, C->jobs_d.as<JobDev<T>>(), num_jobs, C->job_norm_d.as<double>(),
-            C->job_out_d.as<unsigned long long>());
+            C->scalars.as<unsigned long long>() + SC_COUNT);
     HIP_TRY(hipGetLastError());
     return MI355_OK;
 }
@@ -864,11 +918,12 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     const int th = bands ? BandPlain::kRegionH : strips ? (comp ? StripComp::kRegionH : StripPlain::kRegionH) : kTileH;
 
     // Jobs.
-    C->h_jobs.resize(sizeof(JobDev<T>) * num_jobs);
+    const JobLayout layout(sizeof(JobDev<T>), num_jobs);
+    C->h_jobs.resize(layout.bytes);
     JobDev<T>* hj = reinterpret_cast<JobDev<T>*>(C->h_jobs.data());
-    C->h_job_chunk_off.assign(num_jobs + 1, 0);
-    C->h_job_tile_base.assign(num_jobs + 1, 0);
-    C->h_job_vis_off.assign(num_jobs + 1, 0);
+    unsigned long long* h_vis_off = layout.vis_off(C->h_jobs.data());
+    unsigned* h_chunk_off = layout.chunk_off(C->h_jobs.data());
+    unsigned* h_tile_base = layout.tile_base(C->h_jobs.data());
     unsigned long long chunks = 0, tiles = 0, n_total = 0;
     for (int j = 0; j < num_jobs; ++j)
     {
@@ -898,18 +953,18 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         // count is, and overrides it)
         d.visits_per_item = band_visits_per_item(J.num_points);
         hj[j] = d;
-        C->h_job_chunk_off[j] = (unsigned)chunks;
-        C->h_job_tile_base[j] = (unsigned)tiles;
-        C->h_job_vis_off[j] = n_total;
+        h_chunk_off[j] = (unsigned)chunks;
+        h_tile_base[j] = (unsigned)tiles;
+        h_vis_off[j] = n_total;
         chunks += (J.num_points + kSelChunk - 1) / kSelChunk;
         tiles += (unsigned long long)d.ntx * d.nty;
         n_total += J.num_points;
         if (tiles > 0xFFFFFFFFull || chunks > 0xFFFFFFFFull)
             return fail(MI355_ERR_TOO_LARGE, "too many tiles or visibilities in one call");
     }
-    C->h_job_chunk_off[num_jobs] = (unsigned)chunks;
-    C->h_job_tile_base[num_jobs] = (unsigned)tiles;
-    C->h_job_vis_off[num_jobs] = n_total;
+    h_chunk_off[num_jobs] = (unsigned)chunks;
+    h_tile_base[num_jobs] = (unsigned)tiles;
+    h_vis_off[num_jobs] = n_total;
     if (n_total >= 0xFFFFFFFFull)
         return fail(MI355_ERR_TOO_LARGE, "more than 2^32-1 visibilities in one call");
     const unsigned num_tiles = (unsigned)tiles;
@@ -928,20 +983,14 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     const int key_table_bits = std::min(kappa_bits, 32 - tile_bits);
     const int key_table_shift = kappa_bits - key_table_bits;
 
-    TRY(ensure(C, C->jobs_d, C->h_jobs.size()));
-    TRY(ensure(C, C->job_chunk_off_d, (num_jobs + 1) * sizeof(unsigned)));
-    TRY(ensure(C, C->job_tile_base_d, (num_jobs + 1) * sizeof(unsigned)));
-    TRY(ensure(C, C->job_vis_off_d, (num_jobs + 1) * sizeof(unsigned long long)));
-    TRY(ensure(C, C->job_out_d, 3 * num_jobs * sizeof(unsigned long long)));
-    TRY(ensure(C, C->job_bbox_d, num_jobs * sizeof(int4)));
+    TRY(ensure(C, C->jobs_d, layout.bytes));
     TRY(ensure(C, C->job_norm_d, num_jobs * sizeof(double)));
     if (!C->capturing)
-    {
-        HIP_TRY(hipMemcpyAsync(C->jobs_d.p, C->h_jobs.data(), C->h_jobs.size(), hipMemcpyHostToDevice, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->job_chunk_off_d.p, C->h_job_chunk_off.data(), (num_jobs + 1) * sizeof(unsigned), hipMemcpyHostToDevice, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->job_tile_base_d.p, C->h_job_tile_base.data(), (num_jobs + 1) * sizeof(unsigned), hipMemcpyHostToDevice, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->job_vis_off_d.p, C->h_job_vis_off.data(), (num_jobs + 1) * sizeof(unsigned long long), hipMemcpyHostToDevice, C->stream));
-    }
+        HIP_TRY(hipMemcpyAsync(C->jobs_d.p, C->h_jobs.data(), layout.bytes, hipMemcpyHostToDevice,
+                C->stream));
+    const unsigned long long* job_vis_off = layout.vis_off(C->jobs_d.p);
+    const unsigned* job_chunk_off = layout.chunk_off(C->jobs_d.p);
+    const unsigned* job_tile_base = layout.tile_base(C->jobs_d.p);
 
     // Selection.
     TRY(ensure(C, C->meta, n_total * sizeof(int4)));
@@ -954,19 +1003,20 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     TRY(ensure(C, C->part_taps, chunks * sizeof(unsigned long long)));
     TRY(ensure(C, C->part_nonfinite, chunks * sizeof(unsigned long long)));
     TRY(ensure(C, C->part_bbox, chunks * sizeof(int4)));
-    TRY(ensure(C, C->scalars, SC_COUNT * sizeof(unsigned long long)));
+    TRY(ensure(C, C->scalars, scalar_slots(num_jobs) * sizeof(unsigned long long)));
     unsigned long long* sc = C->scalars.as<unsigned long long>();
+    unsigned long long* job_out = sc + SC_COUNT;
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, C->stream,
             reinterpret_cast<unsigned*>(sc), (unsigned long long)(2 * SC_COUNT), 0u);
 
     SelectArgs<TI, TA> sa{};
     sa.uu = uu; sa.vv = vv; sa.ww = ww; sa.vis = vis; sa.weight = weight;
     sa.jobs = C->jobs_d.as<JobDev<T>>(); sa.num_jobs = num_jobs;
-    sa.job_chunk_off = C->job_chunk_off_d.as<unsigned>();
+    sa.job_chunk_off = job_chunk_off;
     sa.num_planes = (int)P; sa.support = C->support_d.as<int>();
     sa.oversample = ov; sa.half_ov = half;
     sa.norm_table = C->norm_table.as<double>();
-    sa.plane_off = C->plane_off_d.as<unsigned>();
+    sa.plane_off = plane_offsets(C, P);
     sa.table_id_shift = table_id_shift;
     sa.tw = tw; sa.th = th;
     sa.lane_cells = lane_cells;
@@ -985,11 +1035,11 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         HIP_TRY(hipGetLastError());
     }
     hipLaunchKernelGGL(k_job_reduce<T>, dim3(num_jobs), dim3(kSelThreads), 0, C->stream,
-            C->jobs_d.as<JobDev<T>>(), C->job_chunk_off_d.as<unsigned>(),
+            C->jobs_d.as<JobDev<T>>(), job_chunk_off,
             C->part_norm.as<double>(), C->part_skipped.as<unsigned long long>(),
             C->part_taps.as<unsigned long long>(), C->part_nonfinite.as<unsigned long long>(),
-            C->part_bbox.as<int4>(), C->job_out_d.as<unsigned long long>(),
-            C->job_bbox_d.as<int4>(), C->job_norm_d.as<double>());
+            C->part_bbox.as<int4>(), job_out,
+            reinterpret_cast<int4*>(sc + job_bbox_slot(num_jobs)), C->job_norm_d.as<double>());
     HIP_TRY(hipGetLastError());
     record(C, EV_SELECT);
 
@@ -999,9 +1049,8 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         TRY(scan_u32(C, C->num_visits.as<unsigned>(), C->visit_off.as<unsigned>(), cnt,
                 n_total, sc + SC_VISITS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
     }
-    unsigned long long host_sc[SC_COUNT];
-    C->h_job_out.resize(3 * num_jobs);
-    C->h_job_bbox.resize(num_jobs);
+    C->h_scalars.resize(scalar_slots(num_jobs));
+    unsigned long long* host_sc = C->h_scalars.data();
     // T_vis sizes the buffers from here on: the exact count of tile visits,
     // or (host-sync-free) an upper bound from the largest support, the
     // kernels reading the exact count on the device.
@@ -1023,20 +1072,20 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     }
     else
     {
-        HIP_TRY(hipMemcpyAsync(host_sc, sc, sizeof(host_sc), hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->h_job_out.data(), C->job_out_d.p, 3 * num_jobs * sizeof(unsigned long long), hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipMemcpyAsync(C->h_job_bbox.data(), C->job_bbox_d.p, num_jobs * sizeof(int4), hipMemcpyDeviceToHost, C->stream));
+        HIP_TRY(hipMemcpyAsync(host_sc, sc, C->h_scalars.size() * sizeof(unsigned long long),
+                hipMemcpyDeviceToHost, C->stream));
         HIP_TRY(hipStreamSynchronize(C->stream));
         if (host_sc[SC_OVERFLOW]) return fail(MI355_ERR_TOO_LARGE, "more than 2^32-1 tile visits in one call");
         T_vis = host_sc[SC_VISITS];
         for (int j = 0; j < num_jobs; ++j)
         {
-            C->stats.num_skipped += C->h_job_out[3 * j];
-            C->stats.num_taps += C->h_job_out[3 * j + 1];
-            num_nonfinite += C->h_job_out[3 * j + 2];
+            C->stats.num_skipped += host_sc[SC_COUNT + 3 * j];
+            C->stats.num_taps += host_sc[SC_COUNT + 3 * j + 1];
+            num_nonfinite += host_sc[SC_COUNT + 3 * j + 2];
         }
         C->stats.num_visits = T_vis;
-        if (before_grid) TRY((*before_grid)(C, C->h_job_bbox.data()));
+        if (before_grid) TRY((*before_grid)(C,
+                reinterpret_cast<const int4*>(host_sc + job_bbox_slot(num_jobs))));
         if (T_vis == 0)
         {
             record(C, EV_BUCKET); record(C, EV_GRID); record(C, EV_MERGE);
@@ -1058,7 +1107,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     }
     hipLaunchKernelGGL(k_emit<T>, dim3(grid_blocks(n_total, 256, 16384)), dim3(256), 0, C->stream,
             C->meta.as<int4>(), C->num_visits.as<unsigned>(), C->visit_off.as<unsigned>(),
-            C->jobs_d.as<JobDev<T>>(), C->job_vis_off_d.as<unsigned long long>(), num_jobs,
+            C->jobs_d.as<JobDev<T>>(), job_vis_off, num_jobs,
             n_total, tw, th, key_table_shift, key_table_bits, orient_bits, C->keys[0].as<unsigned>(),
             C->vals[0].as<unsigned>());
     HIP_TRY(hipGetLastError());
@@ -1111,7 +1160,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         const auto gather = wide ? k_gather_bands<T, double> : k_gather_bands<T, T>;
         hipLaunchKernelGGL(gather, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0, C->stream,
                 svals, C->vrec.as<VisRec<T>>(), skeys, key_table_bits, C->jobs_d.as<JobDev<T>>(),
-                C->job_tile_base_d.as<unsigned>(), num_jobs, sc + SC_VISITS,
+                job_tile_base, num_jobs, sc + SC_VISITS,
                 C->vmeta.as<int4>(), C->vamp.as<T2>());
         HIP_TRY(hipGetLastError());
     }
@@ -1123,39 +1172,40 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         hipLaunchKernelGGL(k_gather_visits<T>, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0,
                 C->stream, svals, C->vrec.as<VisRec<T>>(), run_flag, run_excl,
                 C->run_start.as<unsigned>(), stage_thresholds(C), kStripMaxW, kStripS, skeys,
-                key_table_bits, C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(),
+                key_table_bits, C->jobs_d.as<JobDev<T>>(), job_tile_base,
                 num_jobs, th, table_id_shift == 0 ? noff : 0, ov % 2 == 0 ? ov / 2 : -1,
                 sc + SC_VISITS, C->vmeta.as<int4>(), C->vamp.as<T2>(), C->vlds.as<int>());
         HIP_TRY(hipGetLastError());
     }
 
     // Tiles -> work items.
-    TRY(ensure(C, C->tile_start, num_tiles * sizeof(unsigned)));
-    TRY(ensure(C, C->tile_end, num_tiles * sizeof(unsigned)));
+    TRY(ensure(C, C->tile_bounds, 2ull * num_tiles * sizeof(unsigned)));
+    unsigned* tile_start = C->tile_bounds.as<unsigned>();
+    unsigned* tile_end = tile_start + num_tiles;
     TRY(ensure(C, C->n_items, num_tiles * sizeof(unsigned)));
     TRY(ensure(C, C->n_slots, num_tiles * sizeof(unsigned)));
     TRY(ensure(C, C->item_off, (num_tiles + 1) * sizeof(unsigned)));
     TRY(ensure(C, C->slot_off, (num_tiles + 1) * sizeof(unsigned)));
     const unsigned tb = grid_blocks(num_tiles, 256, 16384);
-    hipLaunchKernelGGL(k_fill_u32, dim3(tb), dim3(256), 0, C->stream, C->tile_start.as<unsigned>(), (unsigned long long)num_tiles, 0u);
-    hipLaunchKernelGGL(k_fill_u32, dim3(tb), dim3(256), 0, C->stream, C->tile_end.as<unsigned>(), (unsigned long long)num_tiles, 0u);
+    hipLaunchKernelGGL(k_fill_u32, dim3(tb), dim3(256), 0, C->stream, tile_start,
+            2ull * num_tiles, 0u);
     hipLaunchKernelGGL(k_tile_bounds, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0, C->stream,
-            skeys, sc + SC_VISITS, key_table_bits, C->tile_start.as<unsigned>(), C->tile_end.as<unsigned>());
+            skeys, sc + SC_VISITS, key_table_bits, tile_start, tile_end);
     const size_t slot_bytes = (size_t)(tw * th) * (wide ? sizeof(double2) : sizeof(T2));
     unsigned long long num_items, num_slots;
     // items of `override` visits, or of the jobs' own sizes (counts for the
     // launches: from the device, or, host-sync-free, from bounds)
     auto make_items = [&](unsigned override) -> int {
         hipLaunchKernelGGL(k_items<T>, dim3(tb), dim3(256), 0, C->stream,
-                C->tile_start.as<unsigned>(), C->tile_end.as<unsigned>(), num_tiles,
-                C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(), num_jobs, override,
+                tile_start, tile_end, num_tiles,
+                C->jobs_d.as<JobDev<T>>(), job_tile_base, num_jobs, override,
                 C->n_items.as<unsigned>(), C->n_slots.as<unsigned>());
         HIP_TRY(hipGetLastError());
         DevCount cnt{nullptr, 1, 0, num_tiles};
-        TRY(scan_u32(C, C->n_items.as<unsigned>(), C->item_off.as<unsigned>(), cnt, num_tiles,
-                sc + SC_ITEMS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
-        TRY(scan_u32(C, C->n_slots.as<unsigned>(), C->slot_off.as<unsigned>(), cnt, num_tiles,
-                sc + SC_SLOTS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
+        const ScanJob scans[2] = {
+            {C->n_items.as<unsigned>(), C->item_off.as<unsigned>(), sc + SC_ITEMS},
+            {C->n_slots.as<unsigned>(), C->slot_off.as<unsigned>(), sc + SC_SLOTS}};
+        TRY(scan_u32(C, scans, 2, cnt, num_tiles, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
         if (C->sync_free)
         {
             // a tile of c visits has ceil(c / V) items, and slots only when that
@@ -1172,7 +1222,8 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         }
         else
         {
-            HIP_TRY(hipMemcpyAsync(host_sc, sc, sizeof(host_sc), hipMemcpyDeviceToHost, C->stream));
+            HIP_TRY(hipMemcpyAsync(host_sc, sc, SC_COUNT * sizeof(unsigned long long),
+                    hipMemcpyDeviceToHost, C->stream));
             HIP_TRY(hipStreamSynchronize(C->stream));
             num_items = host_sc[SC_ITEMS];
             num_slots = host_sc[SC_SLOTS];
@@ -1201,10 +1252,10 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         TRY(ensure(C, C->order_count, kOrderBuckets * sizeof(unsigned)));
         unsigned* first = ordered ? C->order_count.as<unsigned>() : nullptr;
         BandItemArgs ba{C->item_off.as<unsigned>() + num_tiles, C->item_tile.as<unsigned>(),
-                C->item_off.as<unsigned>(), C->slot_off.as<unsigned>(), C->tile_start.as<unsigned>(),
-                C->tile_end.as<unsigned>(), skeys, override, (unsigned)((1ull << key_table_bits) - 1),
+                C->item_off.as<unsigned>(), C->slot_off.as<unsigned>(), tile_start,
+                tile_end, skeys, override, (unsigned)((1ull << key_table_bits) - 1),
                 std::max(0, key_table_bits - bits_for(kOrderBuckets)),
-                C->job_tile_base_d.as<unsigned>(), num_jobs, tw, th};
+                job_tile_base, num_jobs, tw, th};
         const dim3 ib(grid_blocks(num_items, 256, 1024));
         if (ordered)
         {
@@ -1230,14 +1281,14 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     ga.meta = C->meta.as<int4>();
     ga.amp = C->amp.as<T4>();
     ga.visit_vis = svals;
-    ga.tile_start = C->tile_start.as<unsigned>();
-    ga.tile_end = C->tile_end.as<unsigned>();
+    ga.tile_start = tile_start;
+    ga.tile_end = tile_end;
     ga.item_off = C->item_off.as<unsigned>();
     ga.slot_off = C->slot_off.as<unsigned>();
     ga.item_tile = C->item_tile.as<unsigned>();
     ga.d_num_items = reinterpret_cast<const unsigned*>(C->item_off.as<unsigned>() + num_tiles);
     ga.jobs = C->jobs_d.as<JobDev<T>>();
-    ga.job_tile_base = C->job_tile_base_d.as<unsigned>();
+    ga.job_tile_base = job_tile_base;
     ga.num_jobs = num_jobs;
     ga.visits_per_item = vpi;
     ga.scratch = C->scratch.p;
@@ -1343,12 +1394,12 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         if (comp)
             hipLaunchKernelGGL((k_merge<T, double2>), dim3(merge_blocks), dim3(256), 0, C->stream,
                     C->item_off.as<unsigned>(), C->slot_off.as<unsigned>(), num_tiles,
-                    C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(), num_jobs,
+                    C->jobs_d.as<JobDev<T>>(), job_tile_base, num_jobs,
                     tw, th, C->scratch.as<double2>());
         else
             hipLaunchKernelGGL((k_merge<T, T2>), dim3(merge_blocks), dim3(256), 0, C->stream,
                     C->item_off.as<unsigned>(), C->slot_off.as<unsigned>(), num_tiles,
-                    C->jobs_d.as<JobDev<T>>(), C->job_tile_base_d.as<unsigned>(), num_jobs,
+                    C->jobs_d.as<JobDev<T>>(), job_tile_base, num_jobs,
                     tw, th, C->scratch.as<T2>());
         HIP_TRY(hipGetLastError());
     }
@@ -1620,7 +1671,8 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // One job; its norm/skipped totals go to library scratch (not reported).
     TRY(ensure(C, C->in_norm, sizeof(double)));
     TRY(ensure(C, C->in_skipped, sizeof(unsigned long long)));
-    C->h_jobs.resize(sizeof(JobDev<T>));
+    const JobLayout layout(sizeof(JobDev<T>), 1);
+    C->h_jobs.resize(layout.bytes);
     JobDev<T>* hj = reinterpret_cast<JobDev<T>*>(C->h_jobs.data());
     hj->grid = const_cast<T2*>(reinterpret_cast<const T2*>(grid));
     hj->norm = C->in_norm.as<double>();
@@ -1638,12 +1690,11 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     hj->vis_end = N;
     hj->chunk_base = 0;
     const unsigned long long chunks = (N + kSelChunk - 1) / kSelChunk;
-    C->h_job_chunk_off.assign(2, 0);
-    C->h_job_chunk_off[1] = (unsigned)chunks;
-    TRY(ensure(C, C->jobs_d, sizeof(JobDev<T>)));
-    TRY(ensure(C, C->job_chunk_off_d, 2 * sizeof(unsigned)));
-    HIP_TRY(hipMemcpyAsync(C->jobs_d.p, hj, sizeof(JobDev<T>), hipMemcpyHostToDevice, C->stream));
-    HIP_TRY(hipMemcpyAsync(C->job_chunk_off_d.p, C->h_job_chunk_off.data(), 2 * sizeof(unsigned), hipMemcpyHostToDevice, C->stream));
+    unsigned* h_chunk_off = layout.chunk_off(hj);
+    h_chunk_off[0] = 0;
+    h_chunk_off[1] = (unsigned)chunks;
+    TRY(ensure(C, C->jobs_d, layout.bytes));
+    HIP_TRY(hipMemcpyAsync(C->jobs_d.p, hj, layout.bytes, hipMemcpyHostToDevice, C->stream));
     TRY(ensure(C, C->meta, N * sizeof(int4)));
     TRY(ensure(C, C->amp, N * sizeof(T4)));
     TRY(ensure(C, C->num_visits, N * sizeof(unsigned)));
@@ -1657,11 +1708,11 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     sa.vis = nullptr;      // the adjoint needs the selection only, no amplitudes
     sa.tw = kTileW; sa.th = kTileH;   // (tile-visit counts are computed, not used)
     sa.jobs = C->jobs_d.as<JobDev<T>>(); sa.num_jobs = 1;
-    sa.job_chunk_off = C->job_chunk_off_d.as<unsigned>();
+    sa.job_chunk_off = layout.chunk_off(C->jobs_d.p);
     sa.num_planes = (int)P; sa.support = C->support_d.as<int>();
     sa.oversample = ov; sa.half_ov = half;
     sa.norm_table = C->norm_table.as<double>();
-    sa.plane_off = C->plane_off_d.as<unsigned>();
+    sa.plane_off = plane_offsets(C, P);
     sa.table_id_shift = std::max(0, bits_for((unsigned long long)P * noff * noff) - kTableIdBits);
     sa.meta = C->meta.as<int4>(); sa.amp = C->amp.as<T4>();
     sa.num_visits = C->num_visits.as<unsigned>();
@@ -1689,10 +1740,9 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
             TRY(ensure(C, C->vals[b], N * sizeof(unsigned)));
         }
         // the sort's count: N in sc[SC_VISITS] (two 32-bit words)
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, C->stream,
-                reinterpret_cast<unsigned*>(sc + SC_VISITS), 1ull, (unsigned)N);
-        hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, C->stream,
-                reinterpret_cast<unsigned*>(sc + SC_VISITS) + 1, 1ull, 0u);
+        unsigned* count = reinterpret_cast<unsigned*>(sc + SC_VISITS);
+        hipLaunchKernelGGL(k_fill2_u32, dim3(1), dim3(64), 0, C->stream, count, 1ull, count + 1,
+                1ull, (unsigned)N, 0u);
         hipLaunchKernelGGL(k_degrid_keys, dim3(grid_blocks(N, 256, 16384)), dim3(256), 0, C->stream,
                 C->meta.as<int4>(), (unsigned long long)N, tiles_x, (unsigned)ntile,
                 C->keys[0].as<unsigned>(), C->vals[0].as<unsigned>());
@@ -2252,10 +2302,8 @@ MI355_EXPORT int mi355_ctx_get_stats(const mi355_ctx* Cc, mi355_stats* stats)
     {
         // host-sync-free call: read the counts the device kept
         HIP_TRY(hipSetDevice(C->device));
-        unsigned long long sc[SC_COUNT];
-        std::vector<unsigned long long> jo(3 * (size_t)C->deferred_jobs);
-        HIP_TRY(hipMemcpyAsync(sc, C->scalars.p, sizeof(sc), hipMemcpyDeviceToHost, C->stream));
-        HIP_TRY(hipMemcpyAsync(jo.data(), C->job_out_d.p, jo.size() * sizeof(unsigned long long),
+        std::vector<unsigned long long> sc(SC_COUNT + 3 * (size_t)C->deferred_jobs);
+        HIP_TRY(hipMemcpyAsync(sc.data(), C->scalars.p, sc.size() * sizeof(unsigned long long),
                 hipMemcpyDeviceToHost, C->stream));
         HIP_TRY(hipStreamSynchronize(C->stream));
         C->stats.num_points = C->deferred_points;
@@ -2264,8 +2312,8 @@ MI355_EXPORT int mi355_ctx_get_stats(const mi355_ctx* Cc, mi355_stats* stats)
         C->stats.num_skipped = C->stats.num_taps = 0;
         for (int j = 0; j < C->deferred_jobs; ++j)
         {
-            C->stats.num_skipped += jo[3 * j];
-            C->stats.num_taps += jo[3 * j + 1];
+            C->stats.num_skipped += sc[SC_COUNT + 3 * j];
+            C->stats.num_taps += sc[SC_COUNT + 3 * j + 1];
         }
         if (!C->stats_untimed) collect_timing(C);
         C->stats_deferred = false;
