@@ -2,7 +2,7 @@
 //
 // Pipeline, in launch order:
 //   k_expand_tables  kernel stack -> per-(plane, |off_u|, |off_v|) tables
-//   k_norm_table     sum of Re(tap) over each footprint (FP64, serial order)
+//                    and the sum of Re(tap) over each footprint (FP64)
 //   k_select         per-visibility selection record + tile-visit count
 //   k_job_reduce     per-job norm (FP64), num_skipped, tap count, bbox
 //   scan             exclusive prefix sum of visit counts
@@ -34,94 +34,100 @@ namespace gg {
 // zero; the table's row 0 sits table_pad_rows rows into its block.
 // TI: precision of the caller's kernel stack; TA: precision the gridder
 // accumulates in (the tables are stored in TA; float -> double is exact).
-// One wave per table row (pad rows included): the row's table and row index
-// come from one division per row, and its lanes write the row's W taps in
-// order.  Workgroups stride over a plane's rows (blockIdx.y: plane), so a
-// launch needs few workgroups per plane whatever the planes' sizes.
+// One workgroup per plane and b: the tables of all a read the same rows of the
+// stack, so a wave takes a row of them all (pad rows included) and the stack's
+// lines, read with stride ov, come from the second level once and not once per
+// a.
+//
+// The same pass sums the tables: norm_table[p][off_v + H][off_u + H] = sum over
+// the footprint of Re(tap) in double, what one visibility with these (plane,
+// off_u, off_v) adds to the norm per unit weight (the `sum` of
+// oskar_grid_wproj.c:154, :207, :210).  The taps for -off are those for +off in
+// reverse order, so the entries with one pair of magnitudes share a sum.  Lanes
+// take columns, waves rows, then a fixed-order reduction (deterministic, the
+// same for every table layout; agrees with the serial order's double sum to a
+// few ulps).
+//
+// Bound by the tables' stores and the strided reads.  One wave per table row,
+// and a second kernel that summed the stack's taps, took 206 us (FP64, 8192^2),
+// 132 us (2M visibilities on 8192^2) and 17 us (200k on 2048^2) where this takes
+// 119, 91 and 7.
+constexpr int kExpandThreads = 1024;
+constexpr int kExpandA = 4;                    // tables of one sweep
+
 template <typename TI, typename TA>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(kExpandThreads)
 void k_expand_tables(const typename V2<TI>::t* __restrict__ conv,
         int num_planes, int conv_size_half, int oversample, int half_ov,
         const int* __restrict__ support, const unsigned* __restrict__ plane_off,
-        int lane_cells, typename V2<TA>::t* __restrict__ tables)
+        int lane_cells, typename V2<TA>::t* __restrict__ tables, double* __restrict__ norm_table)
 {
+    constexpr int kWaves = kExpandThreads / 64;
+    __shared__ double part[kWaves][kExpandA];
     const size_t plane_len = (size_t)conv_size_half * conv_size_half;
-    const int noff = half_ov + 1;
+    const int noff = half_ov + 1, side = 2 * half_ov + 1;
     const int pad = table_pad_rows(lane_cells);
     const int lane = lane_id();
-    const int wave = (int)(threadIdx.x >> 6), waves = (int)(blockDim.x >> 6);
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int b = (int)blockIdx.x;
     for (int p = blockIdx.y; p < num_planes; p += gridDim.y)
     {
         const int s = support[p];
         const int W = 2 * s + 1;
         const int stride = table_stride(W, lane_cells);
         const int rows = W + 2 * pad;                    // rows of one padded table
-        const int total_rows = rows * noff * noff;
+        const size_t a_step = (size_t)rows * noff * stride;
         const typename V2<TI>::t* src = conv + plane_len * p;
-        typename V2<TA>::t* dst = tables + plane_off[p];
-        for (int rr = blockIdx.x * waves + wave; rr < total_rows; rr += gridDim.x * waves)
+        typename V2<TA>::t* dst = tables + plane_off[p] + (size_t)rows * b * stride;
+        for (int a0 = 0; a0 < noff; a0 += kExpandA)
         {
-            const int tab = rr / rows;
-            const int jj = rr - tab * rows - pad;
-            const int a = tab / noff, b = tab - a * noff;
-            typename V2<TA>::t* out = dst + (size_t)rr * stride;
-            const bool in = jj >= 0 && jj < W;
-            const typename V2<TI>::t* srow =
-                    src + (in ? (size_t)abs(b + oversample * (jj - s)) * conv_size_half : 0);
-            for (int kk = lane; kk < stride; kk += 64)
+            double sum[kExpandA] = {};
+            for (int row = wave; row < rows; row += kWaves)
             {
-                typename V2<TA>::t o;
-                o.x = (TA)0;
-                o.y = (TA)0;
-                if (in && kk < W)
+                const int jj = row - pad;
+                typename V2<TA>::t* out = dst + a0 * a_step + (size_t)row * stride;
+                const bool in = jj >= 0 && jj < W;
+                const typename V2<TI>::t* srow =
+                        src + (in ? (size_t)abs(b + oversample * (jj - s)) * conv_size_half : 0);
+                for (int kk = lane; kk < stride; kk += 64)
                 {
-                    const typename V2<TI>::t v = srow[abs(a + oversample * (kk - s))];
-                    o.x = (TA)v.x;
-                    o.y = (TA)v.y;
+                    const bool tap = in && kk < W;
+                    const int c = oversample * (kk - s) + a0;
+                    #pragma unroll
+                    for (int a = 0; a < kExpandA; ++a)
+                    {
+                        if (a0 + a >= noff) break;
+                        typename V2<TA>::t o;
+                        o.x = (TA)0;
+                        o.y = (TA)0;
+                        if (tap)
+                        {
+                            const typename V2<TI>::t v = srow[abs(c + a)];
+                            o.x = (TA)v.x;
+                            o.y = (TA)v.y;
+                        }
+                        out[a * a_step + kk] = o;
+                        sum[a] += (double)o.x;
+                    }
                 }
-                out[kk] = o;
             }
-        }
-    }
-}
-
-// norm_table[p][off_v + H][off_u + H] = sum over the footprint of Re(tap) in
-// double: what one visibility with these (plane, off_u, off_v) adds to the
-// norm per unit weight (the `sum` of oskar_grid_wproj.c:154, :207, :210).
-// The footprint's taps for -off are those for +off in reverse order (k ->
-// -k), so one wave sums the entry for (|off_u|, |off_v|) -- lanes take
-// columns, rows in order, then a fixed-order wave reduction (deterministic;
-// agrees with the serial order's double sum to a few ulps) -- and writes it
-// to the four entries with those magnitudes.
-template <typename T>
-__global__ __launch_bounds__(256)
-void k_norm_table(const typename V2<T>::t* __restrict__ conv,
-        int num_planes, int conv_size_half, int oversample, int half_ov,
-        const int* __restrict__ support, double* __restrict__ norm_table)
-{
-    const int side = 2 * half_ov + 1, noff = half_ov + 1;
-    const int total = num_planes * noff * noff;
-    const int lane = lane_id();
-    const int nw = gridDim.x * (blockDim.x >> 6);
-    for (int e = blockIdx.x * (blockDim.x >> 6) + (int)(threadIdx.x >> 6); e < total; e += nw)
-    {
-        const int p = e / (noff * noff);
-        const int r = e - p * noff * noff;
-        const int ov = r / noff, ou = r % noff;           // magnitudes
-        const int s = support[p];
-        const typename V2<T>::t* src = conv + (size_t)conv_size_half * conv_size_half * p;
-        double sum = 0.0;
-        for (int j = -s; j <= s; ++j)
-        {
-            const typename V2<T>::t* row = src + (size_t)abs(ov + oversample * j) * conv_size_half;
-            for (int k = -s + lane; k <= s; k += 64)
-                sum += (double)row[abs(ou + oversample * k)].x;
-        }
-        sum = wave_sum(sum);
-        if (lane < 4)
-        {
-            const int sv = (lane & 2) ? -ov : ov, su = (lane & 1) ? -ou : ou;
-            norm_table[(size_t)p * side * side + (size_t)(sv + half_ov) * side + (su + half_ov)] = sum;
+            #pragma unroll
+            for (int a = 0; a < kExpandA; ++a)
+            {
+                const double x = wave_sum(sum[a]);
+                if (lane == 0) part[wave][a] = x;
+            }
+            __syncthreads();
+            if (threadIdx.x < 4 * kExpandA && a0 + (int)(threadIdx.x >> 2) < noff)
+            {
+                const int a = (int)(threadIdx.x >> 2), sign = (int)(threadIdx.x & 3);
+                double x = 0.0;
+                for (int w = 0; w < kWaves; ++w) x += part[w][a];
+                const int sv = (sign & 2) ? -b : b, su = (sign & 1) ? -(a0 + a) : a0 + a;
+                norm_table[(size_t)p * side * side + (size_t)(sv + half_ov) * side +
+                        (su + half_ov)] = x;
+            }
+            __syncthreads();
         }
     }
 }

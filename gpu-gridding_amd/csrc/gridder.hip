@@ -660,20 +660,11 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         HIP_TRY(hipMemcpyAsync(C->support_d.p, C->h_planes.data(), 2 * P * sizeof(int),
                 hipMemcpyHostToDevice, C->stream));
     }
-    {
-        // four rows (waves) per workgroup, at most 16 workgroups per plane
-        const unsigned rows_max = (unsigned)((Wmax + 2 * table_pad_rows(lane_cells)) * noff * noff);
-        dim3 g(grid_blocks(rows_max, 4, 16), (unsigned)std::min<size_t>(P, 65535));
-        hipLaunchKernelGGL((k_expand_tables<TI, TA>), g, dim3(256), 0, C->stream,
-                conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-                plane_offsets(C, P), lane_cells, C->tables.as<T2>());
-        HIP_TRY(hipGetLastError());
-        const unsigned entries = (unsigned)(P * noff * noff);   // (|off_u|, |off_v|) per plane
-        hipLaunchKernelGGL(k_norm_table<TI>, dim3(grid_blocks(entries, 4, 65535)), dim3(256), 0,
-                C->stream, conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-                C->norm_table.as<double>());
-        HIP_TRY(hipGetLastError());
-    }
+    hipLaunchKernelGGL((k_expand_tables<TI, TA>),
+            dim3((unsigned)noff, (unsigned)std::min<size_t>(P, 65535)), dim3(kExpandThreads), 0,
+            C->stream, conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
+            plane_offsets(C, P), lane_cells, C->tables.as<T2>(), C->norm_table.as<double>());
+    HIP_TRY(hipGetLastError());
     C->cache_conv = conv_dev;
     C->cache_prec = prec;
     C->cache_ov = ov;
