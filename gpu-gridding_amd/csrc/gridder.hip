@@ -762,6 +762,15 @@ int radix_sort(mi355_ctx* C, unsigned long long n_bound, const unsigned long lon
         int key_bits, const V* first, int* cur_out)
 {
     C->bk_valid = false;              // (the ping-pong buffers are rewritten)
+    if (n_bound <= (unsigned long long)kSortChunk)
+    {
+        hipLaunchKernelGGL(k_sort_small<V>, dim3(1), dim3(kSortSmallThreads), 0, C->stream,
+                C->keys[0].as<unsigned>(), first ? first : C->vals[0].as<V>(), C->vals[0].as<V>(),
+                d_n, key_bits);
+        HIP_TRY(hipGetLastError());
+        *cur_out = 0;
+        return MI355_OK;
+    }
     const int bits = (key_bits + 8) / 9 < (key_bits + 7) / 8 ? 9 : 8;
     const unsigned radix = 1u << bits;
     const unsigned long long nchunk = (n_bound + kSortChunk - 1) / kSortChunk;
