@@ -1575,12 +1575,12 @@ void k_grid_nonfinite(const typename V2<T>::t* __restrict__ tables,
 // immediate and a block's loads are in flight together.  What binds it is the
 // vector load path (16 bytes per FP32 tap; 41 of its 64 bytes per clock and
 // CU are moved, 1M visibilities of support up to 32 on a 4096^2 grid: 1.44 ms
-// with one tap and one cell of 8 bytes per lane and load, 1.25 ms so; blocks
+// with one tap and one cell of 8 bytes per lane and load, 1.22 ms so; blocks
 // of at most 4 or 5 units, which leave registers for twice the waves, 1.33 and
 // 1.29 ms).  Lanes past the
-// footprint read nothing (out of the buffers' range: zeros) and the half of a
-// pair that lies past its last column is masked, so cells outside the
-// footprint (which may hold anything) never reach a sum.  The visibilities go
+// footprint read nothing (out of the buffers' range: zeros) and the pair of the
+// odd last column is that column and the one before, masked, so that cells
+// outside the footprint are not read.  The visibilities go
 // in the order `order` gives (grid tiles of their centre cells: waves that run
 // together read neighbouring cells), or in index order when it is null.
 // Output per visibility: sum over taps of conj-folded tap * grid cell, times
@@ -1635,13 +1635,20 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
                 const T2* tp = tab + (nv ? W - 8 : 0) * W + tc;
                 const T2* gp = g0 + c0;
                 const int last = c0 + (N - 1) * kUnit + lc * LC;     // column in the last unit
+                // the pair of the last column starts one column earlier: the
+                // cell behind that column may lie behind the grid (offsets
+                // count from one column before the block's, so that none is
+                // negative)
+                const bool early = LC == 2 && last == W - 1;
+                const unsigned eg = early ? 0u : kSize;
+                const unsigned et = early ? (MIR ? 2 * kSize : 0) : kSize;
                 for (int r0 = 0; r0 < W; r0 += 8)
                 {
-                    const __amdgpu_buffer_rsrc_t rt = table_rsrc(tp, 0x7fffffffu);
-                    const __amdgpu_buffer_rsrc_t rg = table_rsrc(gp, 0x7fffffffu);
+                    const __amdgpu_buffer_rsrc_t rt = table_rsrc(tp - 1, 0x7fffffffu);
+                    const __amdgpu_buffer_rsrc_t rg = table_rsrc(gp - 1, 0x7fffffffu);
                     const bool row = r0 + lr < W, end = row && last < W;
-                    const unsigned t0 = row ? to : kOutOfRange, g1 = row ? go : kOutOfRange;
-                    const unsigned tl = end ? to : kOutOfRange, gl = end ? go : kOutOfRange;
+                    const unsigned t0 = row ? to + kSize : kOutOfRange, g1 = row ? go + kSize : kOutOfRange;
+                    const unsigned tl = end ? to + et : kOutOfRange, gl = end ? go + eg : kOutOfRange;
                     Vals c[N], g[N];
                     #pragma unroll
                     for (int u = 0; u < N; ++u)
@@ -1661,11 +1668,10 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
                             const int hk = MIR ? LC - 1 - h : h;
                             T cx = c[u].v[2 * hk], ci = c[u].v[2 * hk + 1] * cj;
                             T gx = g[u].v[2 * h], gy = g[u].v[2 * h + 1];
-                            if (h > 0 && u == N - 1)
+                            if (LC == 2 && h == 0 && u == N - 1)   // (another lane's)
                             {
-                                const bool in = last + h < W;
-                                cx = in ? cx : (T)0; ci = in ? ci : (T)0;
-                                gx = in ? gx : (T)0; gy = in ? gy : (T)0;
+                                cx = early ? (T)0 : cx; ci = early ? (T)0 : ci;
+                                gx = early ? (T)0 : gx; gy = early ? (T)0 : gy;
                             }
                             re[h] = fma(cx, gx, re[h]); re[h] = fma(ci, gy, re[h]);
                             im[h] = fma(cx, gy, im[h]); im[h] = fma(-ci, gx, im[h]);
@@ -1696,7 +1702,16 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
                 default: columns(c0, mirrored, std::integral_constant<int, kMaxUnits>()); return;
                 }
             };
-            if (mt.z & kFlagNegU) footprint(std::true_type());
+            if (LC == 2 && W == 1)
+            {
+                if (lane == 0)
+                {
+                    const T2 c = *tab, g = *g0;
+                    re[0] = fma(c.x, g.x, c.y * cj * g.y);
+                    im[0] = fma(c.x, g.y, -(c.y * cj) * g.x);
+                }
+            }
+            else if (mt.z & kFlagNegU) footprint(std::true_type());
             else footprint(std::false_type());
         }
         if (LC == 2) { re[0] += re[LC - 1]; im[0] += im[LC - 1]; }
