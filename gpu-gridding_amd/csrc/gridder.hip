@@ -262,7 +262,8 @@ struct mi355_ctx
     // host mirrors kept alive across asynchronous uploads
     std::vector<unsigned char> h_jobs;
     std::vector<int> h_planes;
-    std::vector<unsigned long long> h_scalars;   // (a download's)
+    std::vector<unsigned long long> h_scalars;   // (a download's, where h_down is not there)
+    HostBuf h_down;
 
     hipEvent_t ev[EV_COUNT] = {};
     mi355_stats stats = {};
@@ -526,6 +527,7 @@ int init_ctx(mi355_ctx* C, int device)
             g_scratch_addr[device] = ptr;
         }
     }
+    (void)ensure_host(C->h_down, 4096);
     return MI355_OK;
 }
 
@@ -1049,8 +1051,21 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         TRY(scan_u32(C, C->num_visits.as<unsigned>(), C->visit_off.as<unsigned>(), cnt,
                 n_total, sc + SC_VISITS, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
     }
-    C->h_scalars.resize(scalar_slots(num_jobs));
-    unsigned long long* host_sc = C->h_scalars.data();
+    // (pinned: a copy to pageable memory goes through a bounce buffer with waits
+    // of its own; an allocation-free call keeps to what its context has)
+    const size_t down_bytes = scalar_slots(num_jobs) * sizeof(unsigned long long);
+    unsigned long long* host_sc = nullptr;
+    if (!C->sync_free)
+    {
+        if (down_bytes <= C->h_down.cap ||
+                (!C->arena && ensure_host(C->h_down, down_bytes + down_bytes / 2) == MI355_OK))
+            host_sc = static_cast<unsigned long long*>(C->h_down.p);
+        else
+        {
+            C->h_scalars.resize(scalar_slots(num_jobs));
+            host_sc = C->h_scalars.data();
+        }
+    }
     // T_vis sizes the buffers from here on: the exact count of tile visits,
     // or (host-sync-free) an upper bound from the largest support, the
     // kernels reading the exact count on the device.
@@ -1072,8 +1087,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     }
     else
     {
-        HIP_TRY(hipMemcpyAsync(host_sc, sc, C->h_scalars.size() * sizeof(unsigned long long),
-                hipMemcpyDeviceToHost, C->stream));
+        HIP_TRY(hipMemcpyAsync(host_sc, sc, down_bytes, hipMemcpyDeviceToHost, C->stream));
         HIP_TRY(hipStreamSynchronize(C->stream));
         if (host_sc[SC_OVERFLOW]) return fail(MI355_ERR_TOO_LARGE, "more than 2^32-1 tile visits in one call");
         T_vis = host_sc[SC_VISITS];
@@ -2195,6 +2209,7 @@ MI355_EXPORT int mi355_ctx_destroy(mi355_ctx* C)
         release_host(C->h_stage[i]);
         if (C->stage_ev[i]) (void)hipEventDestroy(C->stage_ev[i]);
     }
+    release_host(C->h_down);
     for (int i = 0; i < EV_COUNT; ++i) if (C->ev[i]) (void)hipEventDestroy(C->ev[i]);
     if (C->switch_ev) (void)hipEventDestroy(C->switch_ev);
     delete C;
