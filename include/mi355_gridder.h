@@ -317,9 +317,9 @@ MI355_EXPORT int mi355_grid_wproj_f_batched_graph_dev(mi355_ctx* ctx,
  * outputs (one scratch grid per job; the job table's grids are not
  * touched), first over the gridding kernel / tile geometry (the band
  * kernel where that is the automatic one, 16-column strips on 256x128
- * regions, or 64x64 tiles), work-item size and item grouping, then, for the strip kernel, over the shortest staged run of
- * each support class in turn (tables at most 33, 65, 97, 111 wide), and
- * leaves the fastest settings in the context's options
+ * regions, or 64x64 tiles), work-item size and item grouping, then, for
+ * the strip kernel, over the shortest staged run of each support class in
+ * turn (tables at most 33, 65, 97, 111 wide), and leaves the fastest settings in the context's options
  * (MI355_OPT_GRID_KERNEL, _VISITS_PER_ITEM, _ITEM_GROUP, _MIN_STAGE_RUN,
  * _MIN_STAGE_RUN_W33 .. _W111).  The choice is cached on the context per
  * workload shape (job count, visibility counts, grid sizes, w-planes and
