@@ -60,7 +60,8 @@ __global__ __launch_bounds__(kExpandThreads)
 void k_expand_tables(const typename V2<TI>::t* __restrict__ conv,
         int num_planes, int conv_size_half, int oversample, int half_ov,
         const int* __restrict__ support, const unsigned* __restrict__ plane_off,
-        int lane_cells, typename V2<TA>::t* __restrict__ tables, double* __restrict__ norm_table)
+        int lane_cells, typename V2<TA>::t* __restrict__ tables, unsigned guard, unsigned tail_at,
+        unsigned tail, double* __restrict__ norm_table)
 {
     constexpr int kWaves = kExpandThreads / 64;
     __shared__ double part[kWaves][kExpandA];
@@ -70,6 +71,15 @@ void k_expand_tables(const typename V2<TI>::t* __restrict__ conv,
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int b = (int)blockIdx.x;
+    // the zeros before and behind the tables
+    for (unsigned long long i = (blockIdx.y * (unsigned long long)gridDim.x + blockIdx.x) *
+            kExpandThreads + threadIdx.x; i < (unsigned long long)guard + tail;
+            i += (unsigned long long)gridDim.x * gridDim.y * kExpandThreads)
+    {
+        typename V2<TA>::t z;
+        z.x = z.y = (TA)0;
+        tables[i < guard ? i : tail_at + (i - guard)] = z;
+    }
     for (int p = blockIdx.y; p < num_planes; p += gridDim.y)
     {
         const int s = support[p];
@@ -989,15 +999,6 @@ __global__ void k_fill_u32(unsigned* __restrict__ p, unsigned long long n, unsig
         p[i] = v;
 }
 
-// Two ranges in one launch: a's words to va, b's to vb.
-__global__ void k_fill2_u32(unsigned* __restrict__ a, unsigned long long na,
-        unsigned* __restrict__ b, unsigned long long nb, unsigned va, unsigned vb)
-{
-    for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
-            i < na + nb; i += (unsigned long long)gridDim.x * blockDim.x)
-        if (i < na) a[i] = va; else b[i - na] = vb;
-}
-
 __global__ void k_tile_bounds(const unsigned* __restrict__ keys,
         const unsigned long long* __restrict__ d_n, int key_table_bits,
         unsigned* __restrict__ tile_start, unsigned* __restrict__ tile_end)
@@ -1728,8 +1729,10 @@ void k_degrid(const typename V2<T>::t* __restrict__ tables,
 // Degridding order keys: the 64 x 64 grid tile of each visibility's centre
 // cell (tiles_x per tile row), skipped visibilities under skip_key.
 __global__ void k_degrid_keys(const int4* __restrict__ meta, unsigned long long n, int tiles_x,
-        unsigned skip_key, unsigned* __restrict__ keys, unsigned* __restrict__ vals)
+        unsigned skip_key, unsigned* __restrict__ keys, unsigned* __restrict__ vals,
+        unsigned long long* __restrict__ count)
 {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *count = n;       // (the sort's)
     for (unsigned long long i = blockIdx.x * (unsigned long long)blockDim.x + threadIdx.x;
             i < n; i += (unsigned long long)gridDim.x * blockDim.x)
     {

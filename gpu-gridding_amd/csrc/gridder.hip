@@ -644,14 +644,6 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         return fail(MI355_ERR_TOO_LARGE, "expanded kernel tables exceed 2 GiB");
     TRY(ensure(C, C->tables, (off + tail) * sizeof(T2)));
     C->table_tail = tail;
-    {
-        // zero the guard and the tail (a fill kernel: no memset nodes)
-        const unsigned wpe = sizeof(T2) / 4;
-        hipLaunchKernelGGL(k_fill2_u32, dim3(grid_blocks((guard + tail) * wpe, 256, 1024)), dim3(256),
-                0, C->stream, C->tables.as<unsigned>(), guard * wpe,
-                reinterpret_cast<unsigned*>(C->tables.as<T2>() + off), tail * wpe, 0u, 0u);
-        HIP_TRY(hipGetLastError());
-    }
     TRY(ensure(C, C->norm_table, P * (2 * half + 1) * (2 * half + 1) * sizeof(double)));
     TRY(ensure(C, C->support_d, 2 * P * sizeof(int)));
     C->cache_support.assign(support, support + P);
@@ -665,7 +657,8 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     hipLaunchKernelGGL((k_expand_tables<TI, TA>),
             dim3((unsigned)noff, (unsigned)std::min<size_t>(P, 65535)), dim3(kExpandThreads), 0,
             C->stream, conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-            plane_offsets(C, P), lane_cells, C->tables.as<T2>(), C->norm_table.as<double>());
+            plane_offsets(C, P), lane_cells, C->tables.as<T2>(), (unsigned)guard, (unsigned)off,
+            (unsigned)tail, C->norm_table.as<double>());
     HIP_TRY(hipGetLastError());
     C->cache_conv = conv_dev;
     C->cache_prec = prec;
@@ -1755,13 +1748,9 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
             TRY(ensure(C, C->keys[b], N * sizeof(unsigned)));
             TRY(ensure(C, C->vals[b], N * sizeof(unsigned)));
         }
-        // the sort's count: N in sc[SC_VISITS] (two 32-bit words)
-        unsigned* count = reinterpret_cast<unsigned*>(sc + SC_VISITS);
-        hipLaunchKernelGGL(k_fill2_u32, dim3(1), dim3(64), 0, C->stream, count, 1ull, count + 1,
-                1ull, (unsigned)N, 0u);
         hipLaunchKernelGGL(k_degrid_keys, dim3(grid_blocks(N, 256, 16384)), dim3(256), 0, C->stream,
                 C->meta.as<int4>(), (unsigned long long)N, tiles_x, (unsigned)ntile,
-                C->keys[0].as<unsigned>(), C->vals[0].as<unsigned>());
+                C->keys[0].as<unsigned>(), C->vals[0].as<unsigned>(), sc + SC_VISITS);
         HIP_TRY(hipGetLastError());
         int cur = 0;
         TRY(radix_sort<unsigned>(C, N, sc + SC_VISITS, bits_for(ntile + 1), nullptr, &cur));
