@@ -10,6 +10,7 @@
 #include "gg_grid_bands.hpp"
 #include "gg_weights.hpp"
 #include "gg_image.hpp"
+#include "gg_sizing.hpp"
 #include "gg_status.hpp"
 #include "mi355_gridder.h"
 
@@ -2682,18 +2683,19 @@ MI355_EXPORT int mi355_autotune_f_batched_dev(mi355_ctx* C, size_t P, const int*
     // Trial outputs: a private scratch grid per job (sized for it), norm and
     // count per job, so the caller's outputs are not touched and the trial
     // jobs write as many grids as the real call does.
-    size_t cells = 0;
-    for (int j = 0; j < num_jobs; ++j) cells += (size_t)J[j].grid_size * J[j].grid_size;
+    std::vector<int> sizes;
+    std::vector<size_t> offsets;
+    for (const auto& j : J) sizes.push_back(j.grid_size);
+    const size_t cells = place_grids(sizes, offsets);
     DevBuf tgrid, tnorm, tskip;
     TRY(ensure(C, tgrid, cells * sizeof(float2)));
     TRY(ensure(C, tnorm, (size_t)num_jobs * sizeof(double)));
     TRY(ensure(C, tskip, (size_t)num_jobs * sizeof(unsigned long long)));
-    for (int j = 0, off = 0; j < num_jobs; ++j)
+    for (int j = 0; j < num_jobs; ++j)
     {
-        J[j].grid = tgrid.as<float2>() + off;      // (results are discarded)
+        J[j].grid = tgrid.as<float2>() + offsets[j];      // (results are discarded)
         J[j].norm = tnorm.as<double>() + j;
         J[j].skipped = tskip.as<unsigned long long>() + j;
-        off += J[j].grid_size * J[j].grid_size;
     }
     const bool timing0 = C->timing;
     const unsigned vpi0 = C->visits_per_item, msr0 = C->min_stage_run, ig0 = C->item_group;
