@@ -220,7 +220,6 @@ struct mi355_ctx
     // the last strip- or band-kernel FP32 pass's sorted tile lists (mi355_ctx_get_buckets)
     bool bk_valid = false, bk_bands = false, bk_exact = false;
     int bk_cur = 0, bk_key_table_bits = 0;
-    unsigned long long bk_points = 0;
     unsigned long long bk_count = 0;
     unsigned char* arena = nullptr;
     size_t arena_cap = 0, arena_used = 0;
@@ -1127,7 +1126,6 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     C->bk_valid = f32 && (strips || bands) && !C->sync_free;
     C->bk_bands = bands;
     C->bk_exact = table_id_shift == 0 && key_table_shift == 0;
-    C->bk_points = n_total;
     C->bk_cur = cur;
     C->bk_count = T_vis;
     C->bk_key_table_bits = key_table_bits;
@@ -2361,21 +2359,25 @@ MI355_EXPORT int mi355_ctx_get_buckets(mi355_ctx* C, unsigned long long* count,
         return ok();
     }
     // The band kernel has no runs: what the strip kernel would make of the
-    // same lists (table widths in the band records).
-    std::vector<unsigned> hk(vm.size()), hv(vm.size());
-    std::vector<int4> hm;
+    // same lists.  Where keys stand for several tables each, the visit's table
+    // is told from the band records alone (later calls may have rewritten the
+    // selection records): where its taps start, less the row and column that
+    // k_gather_bands added, to within the column an even start may take off.
+    // Tables lie at least 16 taps apart.
+    using C2 = BandCfg<float, float>;
+    std::vector<unsigned> hk(vm.size());
     HIP_TRY(hipMemcpy(hk.data(), C->keys[C->bk_cur].p, vm.size() * sizeof(unsigned), hipMemcpyDeviceToHost));
-    if (!C->bk_exact && !vm.empty())
-    {
-        hm.resize((size_t)C->bk_points);
-        HIP_TRY(hipMemcpy(hv.data(), C->vals[C->bk_cur].p, vm.size() * sizeof(unsigned), hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(hm.data(), C->meta.p, hm.size() * sizeof(int4), hipMemcpyDeviceToHost));
-    }
+    auto table = [&](const int4& d) {
+        const int W = d.w & 0xffff, top = (d.z << 16) >> 16;
+        const int row = d.y < 0 ? W - 1 + top : -top;
+        const int col = d.w & kBandMirror ? W - C2::kLaneCells : 0;
+        return (int)(((unsigned)d.x - (unsigned)(row * std::abs(d.y))) / C2::kTapBytes) - col;
+    };
     const uint4 thr = stage_thresholds(C);
     for (size_t i = 0, e; i < vm.size(); i = e)
     {
         for (e = i + 1; e < vm.size() && hk[e] == hk[i] &&
-                (C->bk_exact || hm[hv[e]].w == hm[hv[i]].w); ++e) { }
+                (C->bk_exact || std::abs(table(vm[e]) - table(vm[i])) < 8); ++e) { }
         const int W = vm[i].w & 0xffff;
         const unsigned need = W <= 33 ? thr.x : W <= 65 ? thr.y : W <= 97 ? thr.z : thr.w;
         for (size_t q = i; q < e; ++q)
