@@ -1123,7 +1123,8 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     TRY(radix_sort<unsigned>(C, T_vis, sc + SC_VISITS, key_bits, nullptr, &cur));
     const unsigned* skeys = C->keys[cur].as<unsigned>();
     // (for mi355_ctx_get_buckets: where this pass's sorted lists are)
-    C->bk_valid = f32 && (strips || bands) && !C->sync_free;
+    // (compensated bands have regions of their own size, which it does not report)
+    C->bk_valid = f32 && (strips || (bands && !wide)) && !C->sync_free;
     C->bk_bands = bands;
     C->bk_exact = table_id_shift == 0 && key_table_shift == 0;
     C->bk_cur = cur;

@@ -1,6 +1,6 @@
 """What mi355_ctx_get_buckets reports after a band-kernel pass: the lists of
 that pass whatever ran since without touching them, with shortened kernel
-table ids too."""
+table ids too, and nothing where the header promises nothing."""
 import ctypes
 
 import numpy as np
@@ -78,5 +78,23 @@ def test_lists_survive_a_small_degridding(gpu):
             ops.degrid(ks, sub["uu"], sub["vv"], sub["ww"], sub["weight"], c["cell_size_rad"],
                        c["w_scale"], c["grid_size"], grid, ctx=ctx)
             torch.cuda.synchronize()
+    finally:
+        ctx.close()
+
+
+def test_no_lists_of_compensated_bands(gpu):
+    """Compensated bands have regions of 128 x 128 cells: no lists, where keys
+    numbered over 256 x 128 regions are expected."""
+    torch, ops = gpu
+    c = synth.make(0, num_points=20_000, grid_size=1024, num_w_planes=64, max_support=16, seed=6)
+    ctx = _context(torch)
+    try:
+        _grid(torch, ops, c, ctx)
+        assert len(_buckets(ctx)[0]) > 0
+        ctx.set_option(_lib.OPT_COMPENSATED, 1)
+        _grid(torch, ops, c, ctx)
+        with pytest.raises(_lib.GridderError) as e:
+            _buckets(ctx)
+        assert e.value.status == _lib.ERR_INVALID_ARG
     finally:
         ctx.close()
