@@ -2075,11 +2075,14 @@ int image_dev(mi355_ctx* C, int G, const T* grid, double norm, T* image)
         C->fft_double = dbl;
     }
     FFT_TRY(hipfftSetStream(C->fft_plan, C->stream));
-    // The scale goes in before the transform where it cannot push values out
-    // of range, after it otherwise.
+    // The scale goes in before the transform where it is small enough a shift
+    // of the cells' exponents, after it otherwise (a pass over the image more).
+    // The limits leave FP32 cells from 1.3e-26 to 1.6e32 in the normal range
+    // (FP64: 1e-278 to 1e278), and serve norms up to 1.1e12 (1e30).
     const T scale = (T)(norm != 0.0 ? 1.0 / norm : 1.0);
     const T mag = scale < (T)0 ? -scale : scale;
-    const bool early = direct && mag > (T)1e-15 && mag < (T)1e15;
+    const T lo = dbl ? (T)0x1p-100 : (T)0x1p-40, hi = dbl ? (T)0x1p100 : (T)0x1p20;
+    const bool early = direct && mag >= lo && mag <= hi;
     const dim3 pre(grid_blocks(G / 2 + 1, 256, 256), (unsigned)std::min(G, 65535));
     hipLaunchKernelGGL(k_image_pre<T>, pre, dim3(256), 0, C->stream,
             reinterpret_cast<const T2*>(grid), C->fft_work.as<T2>(), (unsigned)G,
