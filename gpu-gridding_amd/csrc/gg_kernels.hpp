@@ -92,7 +92,9 @@ void k_expand_tables(const typename V2<TI>::t* __restrict__ conv,
         for (int a0 = 0; a0 < noff; a0 += kExpandA)
         {
             double sum[kExpandA] = {};
-            for (int row = wave; row < rows; row += kWaves)
+            // (footprint row jj goes to wave jj mod kWaves, pad rows or not, so
+            // that the sums do not depend on the layout)
+            for (int row = (wave + pad) % kWaves; row < rows; row += kWaves)
             {
                 const int jj = row - pad;
                 typename V2<TA>::t* out = dst + a0 * a_step + (size_t)row * stride;
