@@ -1307,7 +1307,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     ga.d_num_runs = sc + SC_RUNS;
     ga.min_stage_run = C->min_stage_run ? C->min_stage_run
                                         : stage_run_default(std::is_same<T, double>::value);
-    if ((strips || bands) && (T_vis + 1) * 4ull > 0xFFFFFFFFull)
+    if (f32 && (strips || bands) && (T_vis + 1) * 4ull > 0xFFFFFFFFull)
         return fail(MI355_ERR_TOO_LARGE, "more than 2^30 tile visits in one call");
     ga.vmeta = C->vmeta.as<int4>();
     ga.vamp = C->vamp.as<T2>();
