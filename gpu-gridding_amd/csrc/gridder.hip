@@ -197,6 +197,7 @@ struct mi355_ctx
     // the device) and stream capture in progress; set by the graph entry.
     bool sync_free = false;
     bool capturing = false;
+    bool coarse_items = false;      // the last pass could not have its own item sizes
     bool stats_deferred = false;    // stats to be read from the device
     unsigned long long deferred_points = 0;
     int deferred_jobs = 0;
@@ -308,21 +309,6 @@ unsigned auto_visits_per_item(unsigned long long num_points, int num_cu)
 // ms at 8; 2.15M-visibility shape 17.0 -> 15.3 ms).
 unsigned stage_run_default(bool fp64_tiles) { return fp64_tiles ? 8u : 3u; }
 
-// Band kernel: visits per work item.  An item is worked on by 32 waves, one
-// per band of 8 rows and column block, so a small call needs small items to
-// fill the chip (kernel and merge, 2,003 visibilities: 157 us with items of
-// 1024 visits, 38 us with 64; 200,000: 269 us with 1024, 221 us with 512),
-// a large one fewer partial regions to merge (13.2M in 24 grids: 23.7 ms with
-// 512, 23.0 ms with 1024, 23.9 ms with 2048).  Up to 65,536 visibilities the
-// size keeps the partial regions below about 200 (50 MiB).
-unsigned band_visits_per_item(unsigned long long num_points)
-{
-    if (num_points > 65536)
-        return num_points < 524288 ? 512u : num_points < (16ull << 20) ? 1024u : 4096u;
-    unsigned v = 64;
-    while (v * 128ull < num_points) v <<= 1;
-    return v;
-}
 // Visibilities from which the band kernel's items go in table order.
 constexpr unsigned long long kBandOrderMin = 524288;
 
@@ -465,13 +451,10 @@ int ensure(mi355_ctx* C, DevBuf& b, size_t bytes)
     return MI355_OK;
 }
 
-// Whether buffer b could hold `bytes` within the static scratch or the
-// workspace cap (a context without either: always).
-bool fits(const mi355_ctx* C, const DevBuf& b, size_t bytes)
+// Whether the static scratch of an allocation-free context has `bytes` left.
+bool arena_holds(const mi355_ctx* C, size_t bytes)
 {
-    if (bytes <= b.cap) return true;
-    if (C->arena) return C->arena_used + 256 + bytes <= C->arena_cap;
-    return !C->max_workspace || C->ws_bytes - b.cap + bytes <= C->max_workspace;
+    return C->arena_used + 256 + bytes <= C->arena_cap;
 }
 
 void release(mi355_ctx* C, DevBuf& b)
@@ -920,6 +903,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     unsigned* h_chunk_off = layout.chunk_off(C->h_jobs.data());
     unsigned* h_tile_base = layout.tile_base(C->h_jobs.data());
     unsigned long long chunks = 0, tiles = 0, n_total = 0;
+    std::vector<JobSize> sizes;
     for (int j = 0; j < num_jobs; ++j)
     {
         const JobHost<TI, TA>& J = jobs[j];
@@ -944,9 +928,7 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         d.vis_begin = n_total;
         d.vis_end = n_total + J.num_points;
         d.chunk_base = (unsigned)chunks;
-        // (the band kernel's own size; the others' is known once the visit
-        // count is, and overrides it)
-        d.visits_per_item = band_visits_per_item(J.num_points);
+        sizes.push_back({J.num_points, (unsigned long long)d.ntx * d.nty});
         hj[j] = d;
         h_chunk_off[j] = (unsigned)chunks;
         h_tile_base[j] = (unsigned)tiles;
@@ -963,6 +945,19 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     if (n_total >= 0xFFFFFFFFull)
         return fail(MI355_ERR_TOO_LARGE, "more than 2^32-1 visibilities in one call");
     const unsigned num_tiles = (unsigned)tiles;
+    // Visits per work item: the option, or automatic, for the band kernel by
+    // job (vpi and the jobs' sizes: items of either, see below).
+    const unsigned vpi = C->visits_per_item ? C->visits_per_item
+                                            : auto_visits_per_item(n_total, C->num_cu);
+    C->stats.visits_per_item = vpi;
+    const size_t slot_bytes = (size_t)(tw * th) * (wide ? sizeof(double2) : sizeof(T2));
+    const int smax = *std::max_element(support, support + P);
+    // (tiles that one footprint can touch)
+    const unsigned long long visits_bound =
+            (unsigned long long)(2 * smax / tw + 2) * (2 * smax / th + 2);
+    std::vector<unsigned> item_sizes;
+    band_item_sizes(sizes, visits_bound, slot_bytes, vpi, item_sizes);
+    for (int j = 0; j < num_jobs; ++j) hj[j].visits_per_item = item_sizes[j];
     const int tile_bits = std::max(1, bits_for(tiles));
     if (tile_bits > 32) return fail(MI355_ERR_TOO_LARGE, "tile id exceeds 32 bits");
     const unsigned long long num_tables = (unsigned long long)P * noff * noff;
@@ -1062,15 +1057,12 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // T_vis sizes the buffers from here on: the exact count of tile visits,
     // or (host-sync-free) an upper bound from the largest support, the
     // kernels reading the exact count on the device.
-    unsigned long long T_vis = 0, num_nonfinite = 0, visits_bound = 0;
+    unsigned long long T_vis = 0, num_nonfinite = 0;
     C->stats.num_points = n_total;
     C->stats_deferred = C->sync_free;
     if (C->sync_free)
     {
         if (before_grid) return fail(MI355_ERR_INVALID_ARG, "host window upload needs host syncs");
-        int smax = 0;
-        for (size_t p = 0; p < P; ++p) smax = std::max(smax, support[p]);
-        visits_bound = (unsigned long long)(2 * smax / tw + 2) * (2 * smax / th + 2);
         T_vis = std::max(1ull, n_total * visits_bound);
         if (T_vis > 0xFFFFFFFFull)
             return fail(MI355_ERR_TOO_LARGE, "tile-visit bound exceeds 2^32-1 (split the call)");
@@ -1100,11 +1092,6 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
             return commit_jobs<T>(C, num_jobs);
         }
     }
-
-    // Visits per work item: the option, or automatic.
-    const unsigned vpi = C->visits_per_item ? C->visits_per_item
-                                            : auto_visits_per_item(n_total, C->num_cu);
-    C->stats.visits_per_item = vpi;
 
     // Emit (tile | table) keys and sort them.
     for (int b = 0; b < 2; ++b)
@@ -1198,7 +1185,6 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
             2ull * num_tiles, 0u);
     hipLaunchKernelGGL(k_tile_bounds, dim3(grid_blocks(T_vis, 256, 65535)), dim3(256), 0, C->stream,
             skeys, sc + SC_VISITS, key_table_bits, tile_start, tile_end);
-    const size_t slot_bytes = (size_t)(tw * th) * (wide ? sizeof(double2) : sizeof(T2));
     unsigned long long num_items, num_slots;
     // items of `override` visits, or of the jobs' own sizes (counts for the
     // launches: from the device, or, host-sync-free, from bounds)
@@ -1215,16 +1201,14 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         TRY(scan_u32(C, scans, 2, cnt, num_tiles, reinterpret_cast<unsigned*>(sc + SC_OVERFLOW), 1));
         if (C->sync_free)
         {
-            // a tile of c visits has ceil(c / V) items, and slots only when that
-            // is 2 or more, i.e. fewer than 2c / V
             num_items = std::min<unsigned long long>(num_tiles, T_vis) + 1;
             num_slots = 1;
             for (int j = 0; j < num_jobs; ++j)
             {
-                const unsigned long long V = override ? override : hj[j].visits_per_item;
+                const unsigned V = override ? override : hj[j].visits_per_item;
                 const unsigned long long c = jobs[j].num_points * visits_bound;
                 num_items += c / V + 1;
-                num_slots += 2 * c / V + 1;
+                num_slots += slot_bound(c, sizes[j].tiles, V);
             }
         }
         else
@@ -1238,16 +1222,30 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         return MI355_OK;
     };
     // The band kernel takes the jobs' own item sizes, unless one is asked for
-    // or their partial regions would not fit a capped workspace.
-    unsigned override = bands && !C->visits_per_item ? 0u : vpi;
+    // or they do not fit: the static scratch of an allocation-free call, a
+    // workspace cap, or the device (a failed allocation; the captured form of
+    // a pass follows its eager run).
+    auto make_room = [&]() -> int {
+        TRY(ensure(C, C->item_tile, num_items * sizeof(unsigned)));
+        if (bands) TRY(ensure(C, C->band_items, num_items * sizeof(BandItem<T>)));
+        return ensure(C, C->scratch, num_slots * slot_bytes);
+    };
+    unsigned override = !bands || C->visits_per_item ||
+            (C->capturing && C->coarse_items) ? vpi : 0u;
+    if (!C->capturing) C->coarse_items = false;
     TRY(make_items(override));
-    if (!override && !fits(C, C->scratch, num_slots * slot_bytes +
+    int room = MI355_ERR_OUT_OF_MEMORY;
+    if (override || !C->arena || arena_holds(C, num_slots * slot_bytes +
             num_items * (sizeof(unsigned) + sizeof(BandItem<T>)) + 8192))
+        room = make_room();
+    if (room == MI355_ERR_OUT_OF_MEMORY && !override)
     {
         override = vpi;
+        C->coarse_items = true;
         TRY(make_items(override));
+        room = make_room();
     }
-    TRY(ensure(C, C->item_tile, num_items * sizeof(unsigned)));
+    TRY(room);
     hipLaunchKernelGGL(k_item_map, dim3(tb), dim3(256), 0, C->stream, C->item_off.as<unsigned>(),
             num_tiles, C->item_tile.as<unsigned>());
     HIP_TRY(hipGetLastError());
@@ -1255,7 +1253,6 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     {
         // in table order where that pays (larger calls)
         const bool ordered = n_total >= kBandOrderMin;
-        TRY(ensure(C, C->band_items, num_items * sizeof(BandItem<T>)));
         TRY(ensure(C, C->order_count, kOrderBuckets * sizeof(unsigned)));
         unsigned* first = ordered ? C->order_count.as<unsigned>() : nullptr;
         BandItemArgs ba{C->item_off.as<unsigned>() + num_tiles, C->item_tile.as<unsigned>(),
@@ -1280,7 +1277,6 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     C->stats.num_items = num_items;
 
     // Grid.
-    TRY(ensure(C, C->scratch, num_slots * slot_bytes));
     GridArgs<T> ga;
     ga.tables = C->tables.as<T2>();
     ga.table_bytes = (unsigned)((C->table_elems + C->table_tail) * sizeof(T2));

@@ -98,7 +98,12 @@ MI355_EXPORT int mi355_ctx_get_stream(mi355_ctx* ctx, void** hip_stream);
 #define MI355_OPT_VISITS_PER_ITEM 1  /* tile visits per work item; 0: automatic
                                         (default): the largest of 8192, 4096,
                                         2048 for which the call has at least 6 x
-                                        that many visibilities per CU, else 1024 */
+                                        that many visibilities per CU, else 1024;
+                                        the band kernel's automatic items are
+                                        smaller (64 to 1024 visits, by job, below
+                                        16M visibilities), except where their
+                                        partial regions do not fit the device or
+                                        the static scratch */
 #define MI355_OPT_COMPENSATED     2  /* 1: TwoSum-compensated LDS accumulation */
 #define MI355_OPT_PHASE_TIMING    3  /* 1: record hipEvents around each phase */
 #define MI355_OPT_CACHE_KERNELS   4  /* 1: reuse prepared kernel tables while the
@@ -279,6 +284,10 @@ MI355_EXPORT int mi355_degrid_wproj_d_dev(mi355_ctx* ctx,
  * another job's are refused (MI355_ERR_INVALID_ARG), since the jobs'
  * outputs are written concurrently.  (main.cpp's blocks, which all add to
  * one grid, are gridded by calling a single-job entry point per block.)
+ * The band kernel splits up to 8 jobs into work items as calls of their own
+ * would be; more jobs take larger items, so that their grids agree with
+ * single calls' to rounding and not bit for bit.  Repeated passes, eager or
+ * captured, are identical.
  * ---------------------------------------------------------------------- */
 typedef struct
 {
