@@ -1221,16 +1221,17 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         }
         return MI355_OK;
     };
-    // The band kernel takes the jobs' own item sizes, unless one is asked for
-    // or they do not fit: the static scratch of an allocation-free call, a
-    // workspace cap, or the device (a failed allocation; the captured form of
-    // a pass follows its eager run).
+    // The band kernel takes the jobs' own item sizes, unless one is asked for,
+    // the workspace is capped (what a capped context holds already must not
+    // decide how a call is split) or they do not fit: the static scratch of an
+    // allocation-free call, or the device (a failed allocation; the captured
+    // form of a pass follows its eager run).
     auto make_room = [&]() -> int {
         TRY(ensure(C, C->item_tile, num_items * sizeof(unsigned)));
         if (bands) TRY(ensure(C, C->band_items, num_items * sizeof(BandItem<T>)));
         return ensure(C, C->scratch, num_slots * slot_bytes);
     };
-    unsigned override = !bands || C->visits_per_item ||
+    unsigned override = !bands || C->visits_per_item || C->max_workspace ||
             (C->capturing && C->coarse_items) ? vpi : 0u;
     if (!C->capturing) C->coarse_items = false;
     TRY(make_items(override));

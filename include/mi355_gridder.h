@@ -101,9 +101,10 @@ MI355_EXPORT int mi355_ctx_get_stream(mi355_ctx* ctx, void** hip_stream);
                                         that many visibilities per CU, else 1024;
                                         the band kernel's automatic items are
                                         smaller (64 to 1024 visits, by job, below
-                                        16M visibilities), except where their
-                                        partial regions do not fit the device or
-                                        the static scratch */
+                                        16M visibilities), except under a
+                                        workspace cap and where their partial
+                                        regions do not fit the device or the
+                                        static scratch */
 #define MI355_OPT_COMPENSATED     2  /* 1: TwoSum-compensated LDS accumulation */
 #define MI355_OPT_PHASE_TIMING    3  /* 1: record hipEvents around each phase */
 #define MI355_OPT_CACHE_KERNELS   4  /* 1: reuse prepared kernel tables while the

@@ -1,7 +1,7 @@
 """How the band kernel's passes are split into work items where their own item
-sizes cannot be had: the static scratch of the allocation-free entry, a device
-without the memory.  Both then take the size of the other kernels, so that
-grids equal those with that size asked for bit for bit, call
+sizes cannot be had: a workspace cap, the static scratch of the allocation-free
+entry, a device without the memory.  All then take the size of the other
+kernels, so that grids equal those with that size asked for bit for bit, call
 after call and replay after replay.
 """
 import ctypes
@@ -52,6 +52,31 @@ def _run(torch, fn, args, ctx):
 def _equal(a, b):
     return all(same_bits(g0, g1) and n0 == n1 and s0 == s1
                for (g0, n0, s0), (g1, n1, s1) in zip(a, b))
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_split_under_a_cap_does_not_depend_on_the_past(gpu, graph):
+    """A cap that the call fits with room to spare, also once a larger call has
+    gone before, and one that holds little more than the call needs: the same
+    split every time."""
+    torch, ops = gpu
+    args = _jobs(torch, ops, 3, 20_000, 1024, 64, 16)
+    larger = _jobs(torch, ops, 3, 60_000, 1024, 64, 16)
+    fn = ops.grid_batched_graph if graph else ops.grid_batched
+    ctx = _context(torch, OPT_VISITS_PER_ITEM=1024)
+    want, items = _run(torch, fn, args, ctx)
+    ctx.close()
+    ctx = _context(torch)
+    assert _run(torch, fn, args, ctx)[1] > items           # (its own sizes are smaller)
+    ctx.close()
+    for cap, calls in ((1 << 30, (args, args, larger, args)), (128 << 20, (args,) * 3)):
+        ctx = _context(torch, OPT_MAX_WORKSPACE=cap)
+        try:
+            for call in calls:
+                got, n = _run(torch, fn, call, ctx)
+                assert call is larger or (n == items and _equal(got, want)), cap
+        finally:
+            ctx.close()
 
 
 def test_static_scratch_takes_the_coarser_split(gpu):
