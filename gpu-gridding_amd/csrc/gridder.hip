@@ -225,17 +225,24 @@ struct mi355_ctx
     unsigned char* arena = nullptr;
     size_t arena_cap = 0, arena_used = 0;
 
-    // prepared kernel tables
+    // prepared kernel tables: a set per layout (table_stride's lane_cells 0, 1
+    // and 2) while they are cached, all of one kernel stack, so that gridding
+    // and degridding, whose kernels read different layouts, do not evict each
+    // other's; else the first set alone
+    struct TableSet
+    {
+        DevBuf tables, norm, planes;          // (planes: supports, then table offsets)
+        bool valid = false;
+        int lane_cells = 0;
+        unsigned long long elems = 0;         // guard + tables (the zero tail follows)
+        unsigned long long tail = 0;
+    };
+    TableSet table_sets[3];
+    TableSet* tab = &table_sets[0];           // the last call's
     const void* cache_conv = nullptr;
-    int cache_prec = 0, cache_ov = 0, cache_csh = 0, cache_lane_cells = 0;
+    int cache_prec = 0, cache_ov = 0, cache_csh = 0;
     std::vector<int> cache_support;
-    bool tables_valid = false;
-    std::vector<unsigned> plane_off;
-    unsigned long long table_elems = 0;   // guard + tables (the zero tail follows)
-    unsigned long long table_tail = 0;
-    int max_support = 0;
 
-    DevBuf tables, norm_table, support_d;   // (support_d: supports, then table offsets)
     DevBuf meta, amp, num_visits, visit_off;
     DevBuf part_norm, part_skipped, part_taps, part_nonfinite, part_bbox;
     DevBuf scan_partial, scalars;
@@ -396,6 +403,40 @@ int wait_ctx_work(mi355_ctx* C)
     return MI355_OK;
 }
 
+void release(mi355_ctx* C, DevBuf& b)
+{
+    if (C->arena)        // (a view into the static scratch: nothing to free)
+    {
+        b.p = nullptr;
+        b.cap = 0;
+        return;
+    }
+    if (b.p) (void)hipFree(b.p);
+    C->ws_bytes -= b.cap;
+    b.p = nullptr;
+    b.cap = 0;
+}
+
+// The cached table sets but the one in use, for a call that needs the memory.
+int drop_idle_tables(mi355_ctx* C)
+{
+    for (auto& t : C->table_sets)
+    {
+        if (&t == C->tab || !t.tables.cap) continue;
+        TRY(wait_ctx_work(C));
+        t.valid = false;
+        release(C, t.tables);
+        release(C, t.norm);
+        release(C, t.planes);
+    }
+    return MI355_OK;
+}
+
+void forget_tables(mi355_ctx* C)
+{
+    for (auto& t : C->table_sets) t.valid = false;
+}
+
 // Grow-only device allocation of a context's buffer b to at least `bytes`.
 // A buffer that grows is freed only after the context's queued work is done
 // (not the whole device's).  The context's workspace cap
@@ -418,6 +459,8 @@ int ensure(mi355_ctx* C, DevBuf& b, size_t bytes)
         C->arena_used = at + bytes;
         return MI355_OK;
     }
+    if (C->max_workspace && C->ws_bytes - b.cap + bytes > C->max_workspace)
+        TRY(drop_idle_tables(C));
     const size_t others = C->ws_bytes - b.cap;
     if (C->max_workspace && others + bytes > C->max_workspace)
         return fail(MI355_ERR_OUT_OF_MEMORY,
@@ -442,6 +485,12 @@ int ensure(mi355_ctx* C, DevBuf& b, size_t bytes)
         if (e != hipSuccess)
         {
             (void)hipGetLastError();
+            TRY(drop_idle_tables(C));
+            e = hipMalloc(&b.p, bytes);
+        }
+        if (e != hipSuccess)
+        {
+            (void)hipGetLastError();
             b.p = nullptr;
             return fail(MI355_ERR_OUT_OF_MEMORY, "device allocation of %zu bytes failed", bytes);
         }
@@ -455,20 +504,6 @@ int ensure(mi355_ctx* C, DevBuf& b, size_t bytes)
 bool arena_holds(const mi355_ctx* C, size_t bytes)
 {
     return C->arena_used + 256 + bytes <= C->arena_cap;
-}
-
-void release(mi355_ctx* C, DevBuf& b)
-{
-    if (C->arena)        // (a view into the static scratch: nothing to free)
-    {
-        b.p = nullptr;
-        b.cap = 0;
-        return;
-    }
-    if (b.p) (void)hipFree(b.p);
-    C->ws_bytes -= b.cap;
-    b.p = nullptr;
-    b.cap = 0;
 }
 
 void record(mi355_ctx* C, Phase p)
@@ -517,7 +552,9 @@ int init_ctx(mi355_ctx* C, int device)
 // Every device buffer a context holds.
 std::vector<DevBuf*> device_buffers(mi355_ctx* C)
 {
-    return {&C->tables, &C->norm_table, &C->support_d, &C->meta,
+    mi355_ctx::TableSet* t = C->table_sets;
+    return {&t[0].tables, &t[0].norm, &t[0].planes, &t[1].tables, &t[1].norm, &t[1].planes,
+        &t[2].tables, &t[2].norm, &t[2].planes, &C->meta,
         &C->amp, &C->num_visits, &C->visit_off, &C->part_norm, &C->part_skipped,
         &C->part_taps, &C->part_nonfinite, &C->part_bbox, &C->scan_partial, &C->scalars,
         &C->keys[0], &C->keys[1],
@@ -587,20 +624,22 @@ int check_grid_args(int grid_size)
 // ---------------------------------------------------------------------------
 // Kernel tables
 // ---------------------------------------------------------------------------
-const unsigned* plane_offsets(const mi355_ctx* C, size_t P) { return C->support_d.as<unsigned>() + P; }
+const unsigned* plane_offsets(const mi355_ctx* C, size_t P) { return C->tab->planes.as<unsigned>() + P; }
 
 template <typename TI, typename TA>
 int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         const typename V2<TI>::t* conv_dev, int lane_cells)
 {
     const int prec = (int)(16 * sizeof(TI) + sizeof(TA));
-    if (!C->sync_free && C->cache_kernels && C->tables_valid && C->cache_conv == conv_dev &&
-            C->cache_prec == prec && C->cache_ov == ov && C->cache_csh == csh &&
-            C->cache_lane_cells == lane_cells &&
-            C->cache_support.size() == P &&
-            std::equal(support, support + P, C->cache_support.begin()))
-        return MI355_OK;
-    C->tables_valid = false;
+    const bool cached = !C->sync_free && C->cache_kernels;
+    const bool same = C->cache_conv == conv_dev && C->cache_prec == prec && C->cache_ov == ov &&
+            C->cache_csh == csh && C->cache_support.size() == P &&
+            std::equal(support, support + P, C->cache_support.begin());
+    if (!cached || !same) forget_tables(C);
+    mi355_ctx::TableSet& t = C->table_sets[cached ? lane_cells : 0];
+    C->tab = &t;
+    if (t.valid && t.lane_cells == lane_cells) return MI355_OK;
+    t.valid = false;
     const int half = (ov + 1) / 2, noff = half + 1;
     int smax = 0;
     for (size_t p = 0; p < P; ++p) smax = std::max(smax, support[p]);
@@ -610,45 +649,42 @@ int prepare_tables(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     // offsets, below 2^31 so that an offset of 2^31 is out of range.
     const unsigned long long Wmax = 2ull * smax + 1;
     const unsigned long long guard = (unsigned long long)kTableGuardRows * Wmax;
-    C->plane_off.resize(P);
+    C->h_planes.assign(support, support + P);
     unsigned long long off = guard;
     for (size_t p = 0; p < P; ++p)
     {
-        C->plane_off[p] = (unsigned)off;
+        C->h_planes.push_back((int)off);
         off += table_elements(1, support + p, ov, lane_cells);
         if (off > 0x7FFFFFFFull)
             return fail(MI355_ERR_TOO_LARGE, "expanded kernel tables exceed 2^31 elements");
     }
-    C->table_elems = off;
-    C->max_support = smax;
+    t.elems = off;
     typedef typename V2<TA>::t T2;
     const unsigned long long tail = std::max(guard, 2ull * kMaxSupport + 1);
     if ((off + tail) * sizeof(T2) > 0x7FFFFFFFull)
         return fail(MI355_ERR_TOO_LARGE, "expanded kernel tables exceed 2 GiB");
-    TRY(ensure(C, C->tables, (off + tail) * sizeof(T2)));
-    C->table_tail = tail;
-    TRY(ensure(C, C->norm_table, P * (2 * half + 1) * (2 * half + 1) * sizeof(double)));
-    TRY(ensure(C, C->support_d, 2 * P * sizeof(int)));
+    TRY(ensure(C, t.tables, (off + tail) * sizeof(T2)));
+    t.tail = tail;
+    TRY(ensure(C, t.norm, P * (2 * half + 1) * (2 * half + 1) * sizeof(double)));
+    TRY(ensure(C, t.planes, 2 * P * sizeof(int)));
     C->cache_support.assign(support, support + P);
-    C->h_planes.assign(support, support + P);
-    for (unsigned o : C->plane_off) C->h_planes.push_back((int)o);
     if (!C->capturing)   // (a captured pipeline reuses what the eager run uploaded)
     {
-        HIP_TRY(hipMemcpyAsync(C->support_d.p, C->h_planes.data(), 2 * P * sizeof(int),
+        HIP_TRY(hipMemcpyAsync(t.planes.p, C->h_planes.data(), 2 * P * sizeof(int),
                 hipMemcpyHostToDevice, C->stream));
     }
     hipLaunchKernelGGL((k_expand_tables<TI, TA>),
             dim3((unsigned)noff, (unsigned)std::min<size_t>(P, 65535)), dim3(kExpandThreads), 0,
-            C->stream, conv_dev, (int)P, csh, ov, half, C->support_d.as<int>(),
-            plane_offsets(C, P), lane_cells, C->tables.as<T2>(), (unsigned)guard, (unsigned)off,
-            (unsigned)tail, C->norm_table.as<double>());
+            C->stream, conv_dev, (int)P, csh, ov, half, t.planes.as<int>(),
+            plane_offsets(C, P), lane_cells, t.tables.as<T2>(), (unsigned)guard, (unsigned)off,
+            (unsigned)tail, t.norm.as<double>());
     HIP_TRY(hipGetLastError());
     C->cache_conv = conv_dev;
     C->cache_prec = prec;
     C->cache_ov = ov;
     C->cache_csh = csh;
-    C->cache_lane_cells = lane_cells;
-    C->tables_valid = true;
+    t.lane_cells = lane_cells;
+    t.valid = true;
     return MI355_OK;
 }
 
@@ -816,7 +852,7 @@ int grid_nonfinite(mi355_ctx* C, unsigned long long count, int num_jobs,
     typedef typename V2<T>::t T2;
     typedef typename V4<T>::t T4;
     hipLaunchKernelGGL(k_grid_nonfinite<T>, dim3(grid_blocks(n_total, 4, 65535)), dim3(256), 0,
-            C->stream, C->tables.as<T2>(), C->meta.as<int4>(), C->amp.as<T4>(),
+            C->stream, C->tab->tables.as<T2>(), C->meta.as<int4>(), C->amp.as<T4>(),
             C->jobs_d.as<JobDev<T>>(), JobLayout(sizeof(JobDev<T>), num_jobs).vis_off(C->jobs_d.p),
             num_jobs, n_total, C->scalars.as<unsigned long long>() + SC_COUNT, lane_cells);
     HIP_TRY(hipGetLastError());
@@ -1003,9 +1039,9 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     sa.uu = uu; sa.vv = vv; sa.ww = ww; sa.vis = vis; sa.weight = weight;
     sa.jobs = C->jobs_d.as<JobDev<T>>(); sa.num_jobs = num_jobs;
     sa.job_chunk_off = job_chunk_off;
-    sa.num_planes = (int)P; sa.support = C->support_d.as<int>();
+    sa.num_planes = (int)P; sa.support = C->tab->planes.as<int>();
     sa.oversample = ov; sa.half_ov = half;
-    sa.norm_table = C->norm_table.as<double>();
+    sa.norm_table = C->tab->norm.as<double>();
     sa.plane_off = plane_offsets(C, P);
     sa.table_id_shift = table_id_shift;
     sa.tw = tw; sa.th = th;
@@ -1279,9 +1315,9 @@ int run_pipeline(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
 
     // Grid.
     GridArgs<T> ga;
-    ga.tables = C->tables.as<T2>();
-    ga.table_bytes = (unsigned)((C->table_elems + C->table_tail) * sizeof(T2));
-    ga.zero_row_byte = (unsigned)(C->table_elems * sizeof(T2));
+    ga.tables = C->tab->tables.as<T2>();
+    ga.table_bytes = (unsigned)((C->tab->elems + C->tab->tail) * sizeof(T2));
+    ga.zero_row_byte = (unsigned)(C->tab->elems * sizeof(T2));
     ga.meta = C->meta.as<int4>();
     ga.amp = C->amp.as<T4>();
     ga.visit_vis = svals;
@@ -1470,15 +1506,16 @@ int select_dev(mi355_ctx* C, size_t P, const int* support, int ov, size_t N,
     if (N && (!uu || !vv || !ww || !out)) return fail(MI355_ERR_INVALID_ARG, "NULL pointer argument");
     if (N == 0) return ok();
     HIP_TRY(hipSetDevice(C->device));
-    TRY(ensure(C, C->support_d, P * sizeof(int)));
+    DevBuf& planes = C->table_sets[0].planes;
+    TRY(ensure(C, planes, P * sizeof(int)));
     C->cache_support.assign(support, support + P);
-    C->tables_valid = false;
-    HIP_TRY(hipMemcpyAsync(C->support_d.p, C->cache_support.data(), P * sizeof(int),
+    forget_tables(C);
+    HIP_TRY(hipMemcpyAsync(planes.p, C->cache_support.data(), P * sizeof(int),
             hipMemcpyHostToDevice, C->stream));
     const TI gs = G * cell;
     hipLaunchKernelGGL(k_select_out<TI>, dim3(grid_blocks(N, 256, 65535)), dim3(256), 0,
             C->stream, uu, vv, ww, (unsigned long long)N, gs, w_scale, G, ov, (int)P,
-            C->support_d.as<int>(), out);
+            planes.as<int>(), out);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(C->stream));
     return ok();
@@ -1628,7 +1665,7 @@ int grid_host(size_t P, const int* support, int ov, int csh, const T* conv,
     const double zero = 0.0;
     HIP_TRY(hipMemcpyAsync(C->in_norm.p, &zero, sizeof(double), hipMemcpyHostToDevice, C->stream));
     // The host conv_func may change between calls at the same address.
-    C->tables_valid = false;
+    forget_tables(C);
     UploadWindow<T> up;
     up.host_grid = grid;
     up.G = G;
@@ -1715,9 +1752,9 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
     sa.tw = kTileW; sa.th = kTileH;   // (tile-visit counts are computed, not used)
     sa.jobs = C->jobs_d.as<JobDev<T>>(); sa.num_jobs = 1;
     sa.job_chunk_off = layout.chunk_off(C->jobs_d.p);
-    sa.num_planes = (int)P; sa.support = C->support_d.as<int>();
+    sa.num_planes = (int)P; sa.support = C->tab->planes.as<int>();
     sa.oversample = ov; sa.half_ov = half;
-    sa.norm_table = C->norm_table.as<double>();
+    sa.norm_table = C->tab->norm.as<double>();
     sa.plane_off = plane_offsets(C, P);
     sa.table_id_shift = std::max(0, bits_for((unsigned long long)P * noff * noff) - kTableIdBits);
     sa.meta = C->meta.as<int4>(); sa.amp = C->amp.as<T4>();
@@ -1754,7 +1791,7 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         order = C->vals[cur].as<unsigned>();
     }
     hipLaunchKernelGGL(k_degrid<T>, dim3(grid_blocks(N, 4, 65535)), dim3(256), 0, C->stream,
-            C->tables.as<T2>(), C->meta.as<int4>(), order, weight, (unsigned long long)N,
+            C->tab->tables.as<T2>(), C->meta.as<int4>(), order, weight, (unsigned long long)N,
             reinterpret_cast<const T2*>(grid), G, apply_weight, reinterpret_cast<T2*>(out));
     HIP_TRY(hipGetLastError());
     return ok();
@@ -2242,7 +2279,7 @@ MI355_EXPORT int mi355_ctx_set_option(mi355_ctx* C, int key, long long value)
         break;
     case MI355_OPT_COMPENSATED: C->compensated = value != 0; break;
     case MI355_OPT_PHASE_TIMING: C->timing = value != 0; break;
-    case MI355_OPT_CACHE_KERNELS: C->cache_kernels = value != 0; C->tables_valid = false; break;
+    case MI355_OPT_CACHE_KERNELS: C->cache_kernels = value != 0; forget_tables(C); break;
     case MI355_OPT_GRID_KERNEL:
         if (value < 0 || value > 2) return fail(MI355_ERR_INVALID_ARG, "grid kernel %lld", value);
         C->grid_kernel = (int)value;
@@ -2435,7 +2472,7 @@ MI355_EXPORT int mi355_grid_wproj_f_dev_noalloc(mi355_ctx* C, size_t P, const in
     Z->item_group = C->item_group;
     Z->timing = C->timing;
     Z->cache_kernels = false;          // (the scratch is shared: tables are rebuilt per call)
-    Z->tables_valid = false;
+    forget_tables(Z);
     if (Z->stream != C->stream) TRY(mi355_ctx_set_stream(Z, C->stream));
     // every buffer is handed out afresh from the start of the scratch
     Z->arena_used = 0;

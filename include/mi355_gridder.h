@@ -108,7 +108,10 @@ MI355_EXPORT int mi355_ctx_get_stream(mi355_ctx* ctx, void** hip_stream);
 #define MI355_OPT_COMPENSATED     2  /* 1: TwoSum-compensated LDS accumulation */
 #define MI355_OPT_PHASE_TIMING    3  /* 1: record hipEvents around each phase */
 #define MI355_OPT_CACHE_KERNELS   4  /* 1: reuse prepared kernel tables while the
-                                        conv_func pointer and shape are unchanged */
+                                        conv_func pointer and shape are unchanged
+                                        (a set for each of the layouts in use, up
+                                        to three; those not in use are given back
+                                        when a call needs the memory) */
 #define MI355_OPT_GRID_KERNEL     5  /* 0: automatic (default): for FP64 the band
                                         kernel (8-row bands with the cells in LDS);
                                         for FP32 and compensated FP32 the band
