@@ -218,6 +218,15 @@ __device__ __forceinline__ double read_lane(double v, int l)
     return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
+// Orders the lanes' accesses of LDS that one wave shares.  The hardware takes a
+// wave's LDS accesses in program order, so that this costs no instruction; the
+// compiler, which sees each lane alone, must not move them across.
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ unsigned long long lanemask_lt()
 {
     return (1ull << lane_id()) - 1ull;

@@ -122,6 +122,7 @@ void k_grid_bands(const GridArgs<TAP> A)
             for (auto& q : z.v) q = (CELL)0;
             for (int i = lane; i < C::kRows * C::kStride; i += 64) cells[8 + i] = z;
         }
+        wave_lds_fence();
 
         // (resources based at the item's records: reads past its last visit
         // return zero, a table of width 0, which meets no band)
@@ -202,6 +203,7 @@ void k_grid_bands(const GridArgs<TAP> A)
                 }
                 #pragma unroll
                 for (int u = 0; u < N; ++u) cell[u * 8] = s[u];
+                wave_lds_fence();        // (the next visit's cells are other lanes')
             };
             auto by_units = [&](int l, int q, auto mirrored) {
                 switch ((q >> 8) & 15)
@@ -260,6 +262,7 @@ void k_grid_bands(const GridArgs<TAP> A)
             for (int r = 0; r < C::kRows; ++r)
                 reinterpret_cast<Word*>(out + r * C::kRegionW)[lane] = cells[8 + r * C::kStride + lane];
         }
+        wave_lds_fence();
     }
 }
 

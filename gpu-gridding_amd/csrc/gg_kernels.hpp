@@ -833,6 +833,7 @@ void k_sort_scatter(const unsigned* __restrict__ keys_in,
             const unsigned prior = valid ? wcnt[wave][d] : 0u;
             rank[r] = prior + before;
             if (valid && before == 0) wcnt[wave][d] = prior + (unsigned)__popcll(peers);
+            wave_lds_fence();           // (the next row's counts, other lanes')
         }
         __syncthreads();
         // The chunk's digits in order: each thread kPer of them.
@@ -946,6 +947,7 @@ void k_sort_small(unsigned* __restrict__ keys, const V* vals_in,
             const unsigned prior = valid ? wcnt[wave][d] : 0u;
             rank[r] = prior + before;
             if (valid && before == 0) wcnt[wave][d] = prior + (unsigned)__popcll(peers);
+            wave_lds_fence();           // (the next row's counts, other lanes')
         }
         __syncthreads();
         unsigned run = 0, mine = 0;
