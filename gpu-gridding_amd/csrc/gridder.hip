@@ -334,17 +334,20 @@ unsigned long long table_elements(size_t P, const int* support, int ov, int lane
 
 // Whether the band kernel takes a pass (tiles: regions of 256 x 128 cells in
 // all its grids).  Not where another kernel or a staging threshold is asked
-// for.  FP64: always (1.13 to 3.3 times the 64x64 staged kernel's speed at
-// supports 16 to 72, 0.2M to 12M visibilities, 32 and 300 planes, 2048^2 and
-// 8192^2 grids).  FP32: where tables serve few visits or are small; the strip
-// kernel, which stages a table once for many visits, stays ahead with wide
-// tables on large grids (support 72: 0.86 to 0.96 of its time at 1M to 8M
-// visibilities and 16384^2, but 1.02 to 1.57 times its speed at 2048^2; support
-// 48 and below: 1.0 to 2.3 times) and where a table serves tens of thousands
-// (support 48, 12M visibilities, 32 planes, 8192^2: 0.88).  Compensated FP32
-// has FP64 cells here and so half the cells a lane: ahead up to the visits
-// per table below (1M visibilities, 128 planes, support 32: 1.58 + 0.16 ms
-// before, 1.36 + 0.08 ms).
+// for.  FP64: always (whole pass 1.01 to 2.8 times as fast as with the 64x64
+// staged kernel at supports 8 to 120, 30k to 2M visibilities, 32 and 256 planes,
+// 2048^2 and 8192^2 grids).  FP32: where tables serve few visits or are small;
+// the strip kernel, which stages a table once for many visits, stays ahead with
+// wide tables on large grids (support 72, 8192^2: 0.88 to 0.96 of the band
+// kernel's time at 1M to 10M visibilities, but 1.02 to 1.5 at 2048^2; support
+// 48: 1.01 to 1.3) and where a table serves tens of thousands (support 48, 10M
+// visibilities, 32 planes, 8192^2: 0.93).  Compensated FP32 has FP64 cells here
+// and so half the cells a lane: strips come ahead earlier, at a number of visits
+// per table that falls with the support, and with wide tables at a number of
+// visibilities (band and strip pass, 8192^2: support 24, 10.4k a table, 3.59 and
+// 3.62 ms; 32, 3.5k, 1.93 and 1.91; 44, 870, 2.73 and 2.85; 48, 870, 3.04 and
+// 3.12; 56, 300k visibilities of 128 planes, 1.47 and 1.64, 1M, 3.72 and 3.66;
+// 72, 100k, 1.01 and 1.19, 300k, 2.14 and 2.16).
 template <typename T>
 bool use_bands(const mi355_ctx* C, size_t P, const int* support, int ov, unsigned long long points,
         unsigned long long tiles)
@@ -369,8 +372,10 @@ bool use_bands(const mi355_ctx* C, size_t P, const int* support, int ov, unsigne
     const unsigned long long noff = (ov + 1) / 2 + 1;
     const unsigned long long per_table = points / ((unsigned long long)P * noff * noff);
     if (comp)
-        return per_table < (smax <= 16 ? 16384u : smax <= 36 ? 2048u : smax <= 48 ? 512u
-                            : smax <= 72 ? 128u : 0u);
+        return smax <= 24 ? per_table < 16384
+                : smax <= 36 ? per_table < 3000
+                : smax <= 48 ? per_table < 1000 && points < 1500000
+                : smax <= 72 && points < (smax <= 60 ? 400000u : 150000u);
     if (tiles < 1024) return true;
     return !(smax > 48 && points >= 1000000) && !(smax > 16 && per_table > 20000);
 }
@@ -879,8 +884,9 @@ struct BeforeGrid
     virtual ~BeforeGrid() {}
 };
 
-// use_bands for a job table: by the largest job, so that a batched pass grids
-// a job as a call of its own would.
+// use_bands for a job table: by the largest job and the largest grid, so that
+// jobs of one size are gridded as calls of their own would be (beside a larger
+// one a job may take that one's kernel).
 template <typename TI, typename TA>
 bool auto_kernel_is_bands(const mi355_ctx* C, size_t P, const int* support, int ov, int num_jobs,
         const JobHost<TI, TA>* jobs)

@@ -1,0 +1,59 @@
+"""Which kernel an automatic FP32 pass takes, plain and compensated, on both
+sides of each line of the rule.  The kernels sum in different orders, so that
+of random data a pass equals one with the strip kernel asked for (by a staging
+threshold that is the automatic one) bit for bit only where it took that kernel.
+"""
+import numpy as np
+import pytest
+
+from mi355_gridding import _lib
+from test_gpu_bands import _case
+
+pytestmark = pytest.mark.gpu
+
+LARGE = 5888          # 23 x 46 regions of 256 x 128: more than 1024
+SMALL = 5632          # 22 x 44: fewer
+
+
+def _grid(torch, ops, c, comp, strips):
+    ctx = _lib.Context(torch.cuda.current_device())
+    try:
+        ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+        ctx.set_option(_lib.OPT_COMPENSATED, comp)
+        ctx.set_option(_lib.OPT_MIN_STAGE_RUN_W33, 6 if strips else 0)
+        ks = ops.KernelStack(c["support"], c["oversample"], c["conv_size_half"], c["conv_func"])
+        d = {k: torch.from_numpy(c[k]).cuda() for k in ("uu", "vv", "ww", "vis", "weight")}
+        G = c["grid_size"]
+        g = torch.zeros((G, G, 2), dtype=torch.float32, device="cuda")
+        norm = torch.zeros(1, dtype=torch.float64, device="cuda")
+        sk = torch.zeros(1, dtype=torch.int64, device="cuda")
+        ops.grid(ks, d["uu"], d["vv"], d["ww"], d["vis"], d["weight"], c["cell_size_rad"],
+                 c["w_scale"], G, g, norm, sk, ctx=ctx)
+        torch.cuda.synchronize()
+        return g
+    finally:
+        ctx.close()
+
+
+# (compensated, grid, largest support, planes, oversampling, visibilities, bands?);
+# oversampling 1: 4 tables a plane, 4: 9
+@pytest.mark.parametrize("comp,G,smax,P,ov,N,bands", [
+    (0, SMALL, 17, 1, 1, 84_000, True), (0, LARGE, 17, 1, 1, 84_000, False),
+    (0, LARGE, 17, 1, 1, 80_000, True), (0, LARGE, 16, 1, 1, 84_000, True),
+    (0, LARGE, 49, 8, 4, 999_999, True), (0, LARGE, 49, 8, 4, 1_000_000, False),
+    (0, SMALL, 49, 8, 4, 1_000_000, True), (0, LARGE, 48, 8, 4, 1_000_000, True),
+    (1, 700, 24, 1, 1, 65_532, True), (1, 700, 24, 1, 1, 65_536, False),
+    (1, 700, 36, 2, 4, 53_999, True), (1, 700, 36, 2, 4, 54_000, False),
+    (1, 700, 37, 2, 4, 17_999, True), (1, 700, 48, 2, 4, 18_000, False),
+    (1, 700, 60, 3, 4, 399_999, True), (1, 700, 60, 3, 4, 400_000, False),
+    (1, 700, 61, 3, 4, 149_999, True), (1, 700, 72, 3, 4, 150_000, False),
+    (1, 900, 73, 3, 4, 2000, False), (1, 900, 72, 3, 4, 2000, True)])
+def test_rule_of_the_automatic_choice(gpu, comp, G, smax, P, ov, N, bands):
+    torch, ops = gpu
+    supports = np.linspace(smax, max(1, smax - 8), P).astype(int).tolist()
+    c = _case(G, ov, supports, N, seed=N % 97)
+    assert max(supports) == smax and len(supports) == P
+    auto = _grid(torch, ops, c, comp, False)
+    strips = _grid(torch, ops, c, comp, True)
+    assert torch.equal(auto, strips) != bands
+    assert (auto - strips).abs().max() <= 1e-4 * strips.abs().max()
