@@ -1,5 +1,6 @@
-"""Which kernel an automatic FP32 pass takes, plain and compensated, on both
-sides of each line of the rule.  The kernels sum in different orders, so that
+"""Which kernel an automatic pass takes: FP32, plain and compensated, on both
+sides of each line of the rule; FP64 with and without a workspace cap; and on
+the shapes that the band kernel is checked on.  The kernels split regions into different items, so that
 of random data a pass equals one with the strip kernel asked for (by a staging
 threshold that is the automatic one) bit for bit only where it took that kernel.
 """
@@ -7,7 +8,7 @@ import numpy as np
 import pytest
 
 from mi355_gridding import _lib
-from test_gpu_bands import _case
+from test_gpu_bands import SUPPORTS, _case, _run
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +58,23 @@ def test_rule_of_the_automatic_choice(gpu, comp, G, smax, P, ov, N, bands):
     strips = _grid(torch, ops, c, comp, True)
     assert torch.equal(auto, strips) != bands
     assert (auto - strips).abs().max() <= 1e-4 * strips.abs().max()
+
+
+@pytest.mark.parametrize("G,ov,supports,n", [(333, 4, SUPPORTS, 3000), (640, 3, SUPPORTS, 2000),
+                                             (130, 1, [0, 1, 2], 4000), (1030, 4, [70], 4000),
+                                             (257, 8, [8, 9], 5000)])
+def test_shapes_of_the_band_checks(gpu, G, ov, supports, n):
+    """(Enough visibilities for several items a region: the kernels add one
+    item's visits in the same order.)"""
+    torch, ops = gpu
+    c = _case(G, ov, supports, n, seed=G)
+    grid0 = np.random.default_rng(1).normal(size=(G, G, 2))
+    for dtype, opts, other in ((torch.float32, {}, dict(OPT_MIN_STAGE_RUN_W33=6)),
+                               (torch.float32, dict(OPT_COMPENSATED=1),
+                                dict(OPT_COMPENSATED=1, OPT_MIN_STAGE_RUN_W33=6)),
+                               (torch.float64, {}, dict(OPT_GRID_KERNEL=2)),
+                               (torch.float64, {}, dict(OPT_MAX_WORKSPACE=4 << 30))):
+        a, an, _ = _run(torch, ops, c, dtype, grid0, **opts)
+        b, bn, _ = _run(torch, ops, c, dtype, grid0, **other)
+        assert not np.array_equal(a, b) and np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
+        assert an == bn
