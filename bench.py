@@ -698,7 +698,11 @@ def main():
                                                 a.no_cpu_baseline)
 
     traffic = None
-    kname = {"strips": "k_grid_strips" if a.config == 2 else "k_grid_bands", "staged": "k_grid_staged", "direct": "k_grid_tiles"}[a.kernel]
+    # (the automatic choice at these sizes: bands, but strips for the 31.4M
+    # workload and wherever a staged-run threshold is given)
+    tile_kernel = a.kernel if a.kernel != "strips" or a.config == 2 or a.min_stage_run else "bands"
+    kname = {"strips": "k_grid_strips", "bands": "k_grid_bands", "staged": "k_grid_staged",
+             "direct": "k_grid_tiles"}[tile_kernel]
     if os.path.exists(TRAFFIC_FILE):
         tr = json.load(open(TRAFFIC_FILE)).get(kname)
         if tr and tr.get("workload") == case["name"]:
@@ -726,7 +730,7 @@ def main():
                    "num_w_planes": case["num_w_planes"], "max_support": case["max_support"],
                    "oversample": case["oversample"],
                    "accumulation": "compensated" if a.compensated else "plain",
-                   "tile_kernel": a.kernel if a.config == 2 or a.kernel != "strips" else "bands",
+                   "tile_kernel": tile_kernel,
                    "visits_per_item": int(phases[-1]["visits_per_item"]) if phases
                    else a.visits_per_item,
                    "min_stage_run": a.min_stage_run or "auto", "item_group": a.item_group},

@@ -1,9 +1,9 @@
 """Which kernel an automatic pass takes: FP32, plain and compensated, on both
 sides of each line of the rule; FP64 with and without a workspace cap; and on
-the shapes that the band kernel is checked on.  The kernels split regions into different items, so that
-of random data a pass equals one with the strip kernel asked for (by a staging
-threshold that is the automatic one) bit for bit only where it took that kernel.
-"""
+the shapes that the band kernel is checked on.  The kernels split regions into
+different items, so that of random data a pass equals one with the strip kernel
+asked for (by a staging threshold that is the automatic one) bit for bit only
+where it took that kernel."""
 import numpy as np
 import pytest
 
