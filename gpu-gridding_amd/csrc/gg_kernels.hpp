@@ -13,7 +13,8 @@
 //   k_grid_tiles     one workgroup per work item, tile in registers (or LDS);
 //                    k_grid_strips, k_grid_staged, k_grid_bands: own headers
 //   k_merge          ordered FP64 sum of partial tiles into the grid
-//   k_degrid         adjoint: one wave per visibility, taps dealt to all lanes
+//   k_degrid_flat, k_degrid   adjoint: one wave per visibility, its taps dealt to
+//                    all lanes
 #pragma once
 
 #include "gg_device.hpp"
@@ -1575,23 +1576,87 @@ void k_grid_nonfinite(const typename V2<T>::t* __restrict__ tables,
 // ===========================================================================
 // Degridding (adjoint)
 // ===========================================================================
-// One wave per visibility, its footprint walked in units of 8 rows x 8 lanes:
-// a lane takes 16 bytes of the table and of the grid at a time (two adjacent
-// complex FP32 values, or one FP64 one), the units of 8 rows side by side in
-// one straight-line block, so that every address but the first is an
-// immediate and a block's loads are in flight together.  What binds it is the
-// vector load path (16 bytes per FP32 tap; 41 of its 64 bytes per clock and
-// CU are moved, 1M visibilities of support up to 32 on a 4096^2 grid: 1.44 ms
-// with one tap and one cell of 8 bytes per lane and load, 1.22 ms so; blocks
-// of at most 4 or 5 units, which leave registers for twice the waves, 1.33 and
-// 1.29 ms).  Lanes past the
-// footprint read nothing (out of the buffers' range: zeros) and the pair of the
-// odd last column is that column and the one before, masked, so that cells
-// outside the footprint are not read.  The visibilities go
-// in the order `order` gives (grid tiles of their centre cells: waves that run
-// together read neighbouring cells), or in index order when it is null.
+// One wave per visibility.  The visibilities go in the order `order` gives (grid
+// tiles of their centre cells: waves that run together read neighbouring
+// cells), or in index order when it is null.
 // Output per visibility: sum over taps of conj-folded tap * grid cell, times
 // the weight when apply_weight (the adjoint of oskar_grid_wproj.c:190-209).
+// Two kernels walk the footprint in two ways, chosen by call (degrid_flat).
+//
+// Flat: the W*W taps are dealt to the 64 lanes in row-major order (lane l takes
+// taps l, l+64, ...: row t / W, column t % W, kept up incrementally), so that
+// every lane works whatever W is and a wave's 64 table reads are one contiguous
+// run.  Few registers, many waves in flight, 4 to 5 lines touched per load of 512
+// bytes: the kernel of calls that fill the chip with small footprints, with wide
+// ones whose tables lie beyond L2, and of all large FP64 calls.
+template <typename T>
+__global__ __launch_bounds__(256)
+void k_degrid_flat(const typename V2<T>::t* __restrict__ tables,
+        const int4* __restrict__ meta, const unsigned* __restrict__ order,
+        const T* __restrict__ weight, unsigned long long n,
+        const typename V2<T>::t* __restrict__ grid, int grid_size, int apply_weight,
+        typename V2<T>::t* __restrict__ out)
+{
+    typedef typename V2<T>::t T2;
+    const int lane = lane_id();
+    const unsigned long long nw = (unsigned long long)gridDim.x * (blockDim.x >> 6);
+    const unsigned long long w0 = (unsigned long long)blockIdx.x * (blockDim.x >> 6) +
+            (unsigned)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    for (unsigned long long q = w0; q < n; q += nw)
+    {
+        const unsigned long long i = order ? (unsigned long long)ld_const(order, q) : q;
+        const int4 mt = ld_const(meta, i);
+        T re = (T)0, im = (T)0;
+        if (!(mt.z & kFlagSkip))
+        {
+            const int s = meta_support(mt.z);
+            const int W = 2 * s + 1;
+            const int n2 = W * W;
+            const bool neg_u = mt.z & kFlagNegU, neg_v = mt.z & kFlagNegV;
+            const T cj = (mt.z & kFlagConj) ? (T)-1 : (T)1;
+            // 64 taps further on: dr rows and dc columns (one more row when
+            // the column passes W)
+            const int dr = 64 / W, dc = 64 - dr * W;
+            int r = lane / W, c = lane - (lane / W) * W;
+            const T2* tab = tables + (unsigned)mt.w;                 // table row 0
+            const T2* g0 = grid + (size_t)(mt.y - s) * grid_size + (mt.x - s);
+            for (int t = lane; t < n2; t += 64)
+            {
+                const int tr = neg_v ? W - 1 - r : r;
+                const int tc = neg_u ? W - 1 - c : c;
+                const T2 cv = tab[tr * W + tc];
+                const T2 g = g0[(unsigned)r * (unsigned)grid_size + (unsigned)c];
+                const T ci = cv.y * cj;
+                re = fma(cv.x, g.x, re); re = fma(ci, g.y, re);
+                im = fma(cv.x, g.y, im); im = fma(-ci, g.x, im);
+                r += dr;
+                c += dc;
+                if (c >= W) { c -= W; ++r; }
+            }
+        }
+        re = wave_sum(re);
+        im = wave_sum(im);
+        if (lane == 0)
+        {
+            const T w = apply_weight ? weight[i] : (T)1;
+            T2 v; v.x = re * w; v.y = im * w;
+            out[i] = v;
+        }
+    }
+}
+
+// Units: the footprint walked in units of 8 rows x 8 lanes, 16 bytes of the table
+// and of the grid a lane at a time (two adjacent complex FP32 values, or one FP64
+// one), the units of 8 rows side by side in one straight-line block, so that
+// every address but the first is an immediate and a block's loads are in flight
+// together: half of the loads in FP32 and a few round trips per footprint where
+// the flat walk has one per 64 taps, but up to 16 lines per load and registers
+// for half of the waves (blocks of at most 4 or 5 units, which leave room for
+// twice the waves, 1.33 and 1.29 ms where these take 1.22: 1M visibilities of
+// support up to 32 on a 4096^2 grid; flat 1.44).  Lanes past the footprint read
+// nothing (out of the buffers' range: zeros) and the pair of the odd last column
+// is that column and the one before, masked, so that cells outside the footprint
+// are not read.
 constexpr unsigned kOutOfRange = 0x80000000u;
 
 template <typename T>

@@ -1700,6 +1700,27 @@ int grid_host(size_t P, const int* support, int ov, int csh, const T* conv,
 // ---------------------------------------------------------------------------
 // Degridding (adjoint), device pointers.
 // ---------------------------------------------------------------------------
+// Whether a call's footprints are walked flat.  In units a footprint takes few
+// round trips, which wins wherever waves are too few to hide them: small calls
+// (support 72: 0.26 to 0.9 of the flat kernel's time at 300 to 30,000
+// visibilities), and FP32 footprints of supports 12 to 56, whose loads it halves
+// (1M visibilities, 16 planes, 2048^2: support 14 0.74 and 0.91 ms, 32 0.92 and
+// 1.16).  Calls that fill the chip are faster flat with small footprints (support
+// 3: 0.28 ms flat, 0.48 in units; planes of supports 4 to 16: 1.11 and 1.17 at 2M,
+// but all of support 16, 1.14 and 1.00), with wide ones only where the tables are
+// beyond L2 (all of support 72, 16 planes: 1.20 and 1.52; 4 planes, 8 MiB of
+// tables, support 80: 1.25 and 1.14), and in FP64, whose loads units do not halve
+// (support 64, 72k: 3.4 and 4.9 ms; planes of supports 4 to 48, 300k: 0.84).
+template <typename T>
+bool degrid_flat(size_t n, size_t P, const int* support, unsigned long long table_bytes)
+{
+    const auto s = std::minmax_element(support, support + P);
+    const int lo = *s.first, hi = *s.second;
+    if (sizeof(T) == 8) return n >= 100000 || (n >= 30000 && hi >= 48) || (n >= 2000 && lo >= 32);
+    return (n >= 100000 && hi <= 18 && lo <= 11) ||
+            (n >= 4000 && lo >= 57 && table_bytes >= (16ull << 20));
+}
+
 template <typename T>
 int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         const T* conv, size_t N, const T* uu, const T* vv, const T* ww,
@@ -1796,7 +1817,8 @@ int degrid_dev(mi355_ctx* C, size_t P, const int* support, int ov, int csh,
         TRY(radix_sort<unsigned>(C, N, sc + SC_VISITS, bits_for(ntile + 1), nullptr, &cur));
         order = C->vals[cur].as<unsigned>();
     }
-    hipLaunchKernelGGL(k_degrid<T>, dim3(grid_blocks(N, 4, 65535)), dim3(256), 0, C->stream,
+    hipLaunchKernelGGL((degrid_flat<T>(N, P, support, C->tab->elems * sizeof(T2)) ?
+            k_degrid_flat<T> : k_degrid<T>), dim3(grid_blocks(N, 4, 65535)), dim3(256), 0, C->stream,
             C->tab->tables.as<T2>(), C->meta.as<int4>(), order, weight, (unsigned long long)N,
             reinterpret_cast<const T2*>(grid), G, apply_weight, reinterpret_cast<T2*>(out));
     HIP_TRY(hipGetLastError());
