@@ -332,16 +332,17 @@ unsigned long long table_elements(size_t P, const int* support, int ov, int lane
     return n;
 }
 
-// Whether the band kernel takes a pass (tiles: regions of 256 x 128 cells in
-// all its grids).  Not where another kernel or a staging threshold is asked
+// Whether the band kernel takes a pass (points, tiles: visibilities and regions
+// of 256 x 128 cells of its largest job; all_points: visibilities of all).  Not where another kernel or a staging threshold is asked
 // for.  FP64: always (whole pass 1.01 to 2.8 times as fast as with the 64x64
 // staged kernel at supports 8 to 120, 30k to 2M visibilities, 32 and 256 planes,
 // 2048^2 and 8192^2 grids).  FP32: where tables serve few visits or are small;
 // the strip kernel, which stages a table once for many visits, stays ahead with
 // wide tables on large grids (support 72, 8192^2: 0.88 to 0.96 of the band
 // kernel's time at 1M to 10M visibilities, but 1.02 to 1.5 at 2048^2; support
-// 48: 1.01 to 1.3) and where a table serves tens of thousands (support 48, 10M
-// visibilities, 32 planes, 8192^2: 0.93).  Compensated FP32 has FP64 cells here
+// 48: 1.01 to 1.3), from 1M visibilities in one job or 3M in all (24 jobs of
+// 200,000, support 72, 8192^2: 25.2 and 27.8 ms), and where a table serves tens
+// of thousands (support 48, 10M visibilities, 32 planes, 8192^2: 0.93).  Compensated FP32 has FP64 cells here
 // and so half the cells a lane: strips come ahead earlier, at a number of visits
 // per table that falls with the support, and with wide tables at a number of
 // visibilities (band and strip pass, 8192^2: support 24, 10.4k a table, 3.59 and
@@ -350,7 +351,7 @@ unsigned long long table_elements(size_t P, const int* support, int ov, int lane
 // 72, 100k, 1.01 and 1.19, 300k, 2.14 and 2.16).
 template <typename T>
 bool use_bands(const mi355_ctx* C, size_t P, const int* support, int ov, unsigned long long points,
-        unsigned long long tiles)
+        unsigned long long all_points, unsigned long long tiles)
 {
     constexpr bool f32 = std::is_same<T, float>::value;
     if (C->grid_kernel != 0 || C->min_stage_run || C->msr_class[0] || C->msr_class[1] ||
@@ -377,7 +378,8 @@ bool use_bands(const mi355_ctx* C, size_t P, const int* support, int ov, unsigne
                 : smax <= 48 ? per_table < 1000 && points < 1500000
                 : smax <= 72 && points < (smax <= 60 ? 400000u : 150000u);
     if (tiles < 1024) return true;
-    return !(smax > 48 && points >= 1000000) && !(smax > 16 && per_table > 20000);
+    return !(smax > 48 && points >= 1000000) && !(smax > 60 && all_points >= 3000000) &&
+            !(smax > 16 && per_table > 20000);
 }
 
 // The strip kernel's thresholds per support class (tables at most 33, 65,
@@ -891,14 +893,15 @@ template <typename TI, typename TA>
 bool auto_kernel_is_bands(const mi355_ctx* C, size_t P, const int* support, int ov, int num_jobs,
         const JobHost<TI, TA>* jobs)
 {
-    unsigned long long points = 0, regions = 0;
+    unsigned long long points = 0, all = 0, regions = 0;
     for (int j = 0; j < num_jobs; ++j)
     {
+        all += jobs[j].num_points;
         const unsigned long long G = (unsigned long long)std::max(jobs[j].grid_size, 0);
         points = std::max(points, jobs[j].num_points);
         regions = std::max(regions, ((G + 255) / 256) * ((G + 127) / 128));
     }
-    return use_bands<TA>(C, P, support, ov, points, regions);
+    return use_bands<TA>(C, P, support, ov, points, all, regions);
 }
 
 template <typename TI, typename TA>

@@ -78,3 +78,35 @@ def test_shapes_of_the_band_checks(gpu, G, ov, supports, n):
         b, bn, _ = _run(torch, ops, c, dtype, grid0, **other)
         assert not np.array_equal(a, b) and np.abs(a - b).max() <= 1e-5 * np.abs(b).max()
         assert an == bn
+
+
+@pytest.mark.parametrize("points,smax,bands", [(333_333, 61, True), (333_334, 61, False),
+                                               (333_334, 60, True)])
+def test_rule_for_many_jobs_of_wide_footprints(gpu, points, smax, bands):
+    """9 jobs on large grids: 3 million visibilities in all are the line for
+    supports above 60, below that of each job (1 million)."""
+    torch, ops = gpu
+    c = _case(LARGE, 4, [smax, 3], points, seed=8)
+    ks = ops.KernelStack(c["support"], c["oversample"], c["conv_size_half"], c["conv_func"])
+    d = {k: torch.from_numpy(c[k]).cuda() for k in ("uu", "vv", "ww", "vis", "weight")}
+    cat = {k: torch.cat([v] * 9) for k, v in d.items()}
+    norm = torch.zeros(9, dtype=torch.float64, device="cuda")
+    sk = torch.zeros(9, dtype=torch.int64, device="cuda")
+    grids = []
+    for strips in (False, True):
+        g = torch.zeros((9, LARGE, LARGE, 2), dtype=torch.float32, device="cuda")
+        jobs = [dict(vis_offset=j * points, num_points=points, cell_size_rad=c["cell_size_rad"],
+                     w_scale=c["w_scale"], grid_size=LARGE, grid=g[j], norm=norm[j:j + 1],
+                     num_skipped=sk[j:j + 1]) for j in range(9)]
+        ctx = _lib.Context(torch.cuda.current_device())
+        try:
+            ctx.set_stream(torch.cuda.current_stream().cuda_stream)
+            ctx.set_option(_lib.OPT_MIN_STAGE_RUN_W33, 6 if strips else 0)
+            ops.grid_batched(ks, jobs, cat["uu"], cat["vv"], cat["ww"], cat["vis"], cat["weight"],
+                             ctx=ctx)
+            torch.cuda.synchronize()
+        finally:
+            ctx.close()
+        grids.append(g)
+    assert torch.equal(grids[0], grids[1]) != bands
+    assert (grids[0] - grids[1]).abs().max() <= 1e-4 * grids[1].abs().max()
